@@ -96,7 +96,7 @@ __global__ __launch_bounds__(512) void assign_rc_kernel(const AssignRC a) {
         for (int k = 0; k < UL; ++k) {
             if (nvalid[k] <= 0) continue;
             char* p = plan.out_ptr + int64_t(coff<RANK, true>(plan.cst[kMaxLeaves], idxs[k], j0s[k])) * esz;
-            if (S::out_mode == LM_CONTIG && nvalid[k] == V) {  // rows 16-byte aligned: vector stores
+            if (S::out_mode == LM_CONTIG && nvalid[k] == V) {  // a whole unit: vector stores
                 store_vec_rt(out_nt(plan), p, esz, odt, R[k][S::result_reg]);
             } else {
 #pragma unroll

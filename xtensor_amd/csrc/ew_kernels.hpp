@@ -49,11 +49,20 @@ __device__ __forceinline__ void spec_unit(const P& plan, uint32_t u) {
     }
 }
 
+// Workgroup b of g runs on XCD b % 8.  With `runs`, the work of that group is
+// numbered so that each XCD's groups are consecutive (a bijection of [0, g)).
+__device__ __forceinline__ uint32_t xcd_block(uint32_t runs) {
+    const uint32_t b = blockIdx.x;
+    if (!runs) return b;
+    const uint32_t x = b & 7u, q = gridDim.x >> 3, r = gridDim.x & 7u;
+    return x * q + min(x, r) + (b >> 3);
+}
+
 template <int V, int NR, class S, int RANK>
 __global__ __launch_bounds__(256) void ew_spec_kernel(const EwPlan plan) {
     const uint32_t nunits = uint32_t(plan.units);
     const uint32_t step = gridDim.x * 256u;
-    for (uint32_t u = blockIdx.x * 256u + threadIdx.x; u < nunits; u += step) spec_unit<V, NR, S, RANK>(plan, u);
+    for (uint32_t u = xcd_block(plan.xcd_runs) * 256u + threadIdx.x; u < nunits; u += step) spec_unit<V, NR, S, RANK>(plan, u);
 }
 
 // UPT units per thread (u, u + 256, ...: every wave access stays one

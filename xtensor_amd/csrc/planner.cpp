@@ -564,6 +564,36 @@ struct Dim {
 };
 }  // namespace
 
+// Views of one array shifted against each other (a stencil) read the same
+// cache lines from several leaves.  Such leaves keep the default cache policy,
+// and the launch gives each of the 8 XCDs one contiguous run of workgroups, so
+// that the rows a workgroup shares with its neighbours are in its own L2.
+static void share_lines(EwPlan* p) {
+    p->xcd_runs = 0;
+    struct Span { uintptr_t lo, hi; };
+    Span sp[kMaxLeaves];
+    for (int l = 0; l < p->prog.nleaves; ++l) {
+        const LeafView& v = p->leaves[l];
+        sp[l] = Span{0, 0};
+        if (lm_base(v.mode) == LM_GATHER || lm_base(v.mode) == LM_BCAST) continue;
+        int64_t lo = 0, hi = 0;
+        for (int k = 0; k < p->rank; ++k) {
+            const int64_t ext = (p->shape[k] - 1) * v.stride[k];
+            (ext < 0 ? lo : hi) += ext;
+        }
+        const int esz = dtype_size(v.dtype);
+        sp[l].lo = reinterpret_cast<uintptr_t>(v.ptr) + uintptr_t(lo * esz);
+        sp[l].hi = reinterpret_cast<uintptr_t>(v.ptr) + uintptr_t((hi + 1) * esz);
+    }
+    for (int a = 0; a < p->prog.nleaves; ++a)
+        for (int b = a + 1; b < p->prog.nleaves; ++b) {
+            if (sp[a].hi <= sp[b].lo || sp[b].hi <= sp[a].lo) continue;
+            p->leaves[a].mode &= ~LM_NT;
+            p->leaves[b].mode &= ~LM_NT;
+            p->xcd_runs = 1;
+        }
+}
+
 EwPlan plan_assign(const xg_expr* e, const xg_tensor* out, int V) {
     if (!out || out->ndim < 0 || out->ndim > XG_MAX_RANK || out->dtype < 0 || out->dtype >= XG_NUM_DTYPES)
         raise(XG_INVALID_ARGUMENT, "malformed output tensor");
@@ -654,17 +684,21 @@ EwPlan plan_assign(const xg_expr* e, const xg_tensor* out, int V) {
     for (int k = 0; k < rank; ++k) p.div[k] = make_fastdiv(uint32_t(std::min<int64_t>(merged[size_t(k)].n, 0xffffffff)));
     int osz = dtype_size(out->dtype);
     p.out_ptr = static_cast<char*>(out->data) + out_off * osz;
-    auto aligned = [&](const char* ptr, int esz, int64_t inner_stride, const int64_t* strides) {
-        if (inner_stride != 1) return false;
-        if (reinterpret_cast<uintptr_t>(ptr) % uintptr_t(esz * V) != 0) return false;
-        for (int k = 0; k + 1 < rank; ++k)
-            if (strides[k] % V != 0) return false;
-        return true;
+    // wide accesses need the elements side by side, at element addresses
+    auto contig = [&](const char* ptr, int esz, int64_t inner_stride) {
+        return inner_stride == 1 && reinterpret_cast<uintptr_t>(ptr) % uintptr_t(esz) == 0;
     };
-    p.out_mode = aligned(p.out_ptr, osz, p.out_stride[rank - 1], p.out_stride) ? LM_CONTIG : LM_STRIDED;
-    if (g_nt_stores && int64_t(total) * osz >= kNtMinBytes) p.out_mode |= LM_NT;
+    p.out_mode = contig(p.out_ptr, osz, p.out_stride[rank - 1]) ? LM_CONTIG : LM_STRIDED;
+    // non-temporal stores need rows that start on 16-byte boundaries: a row at
+    // an odd element starts and ends every wave's kilobyte inside a granule,
+    // which a non-temporal store writes in part, while plain stores meet in the
+    // L2 (the float64 [3001, 4099] stencil: 78.7 us a call with this hint and
+    // non-temporal loads of its shifted views, 72.0 us with neither)
+    bool rows16 = reinterpret_cast<uintptr_t>(p.out_ptr) % 16 == 0;
+    for (int k = 0; k + 1 < rank; ++k) rows16 = rows16 && (p.out_stride[k] * osz) % 16 == 0;
+    if (g_nt_stores && rows16 && int64_t(total) * osz >= kNtMinBytes) p.out_mode |= LM_NT;
     p.fill_zero = 0;
-    if (g_fill_granules && lm_base(p.out_mode) == LM_CONTIG && rank >= 2 &&
+    if (g_fill_granules && rows16 && lm_base(p.out_mode) == LM_CONTIG && rank >= 2 &&
         int64_t(total) * osz >= kNtMinBytes && p.out_stride[rank - 2] != inner) {
         // rows apart: a row whose bytes do not start and end on 64-byte
         // boundaries shares its edge granules with memory this launch leaves alone
@@ -691,9 +725,10 @@ EwPlan plan_assign(const xg_expr* e, const xg_tensor* out, int V) {
         }
         max_off = std::max(max_off, lmax);
         int64_t is = lv.stride[rank - 1];
-        lv.mode = is == 0 ? LM_BCAST : aligned(lv.ptr, esz, is, lv.stride) ? LM_CONTIG : LM_STRIDED;
+        lv.mode = is == 0 ? LM_BCAST : contig(lv.ptr, esz, is) ? LM_CONTIG : LM_STRIDED;
         if (lv.mode != LM_BCAST && streams(lv.stride, p.shape, rank, esz)) lv.mode |= LM_NT;
     }
+    share_lines(&p);
     p.index64 = max_off >= (int64_t(1) << 31) ? 1 : 0;
     p.compact = (!p.index64 && rank <= 4) ? 1 : 0;
     if (p.compact) {

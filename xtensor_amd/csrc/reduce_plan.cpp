@@ -528,11 +528,10 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
         lv.ptr = static_cast<const char*>(tl.data) + leaf_off[size_t(pl)] * esz;
         lv.dtype = tl.dtype;
         int64_t lmax = 0;
-        bool al = reinterpret_cast<uintptr_t>(lv.ptr) % uintptr_t(esz * V) == 0;
+        const bool al = reinterpret_cast<uintptr_t>(lv.ptr) % uintptr_t(esz) == 0;  // wide loads at element addresses
         for (int k = 0; k < p.rank; ++k) {
             lv.stride[k] = order[size_t(k)].leaf[pl];
             lmax += (std::max<int64_t>(order[size_t(k)].n, 1) - 1) * std::abs(lv.stride[k]);
-            if (k + 1 < p.rank && lv.stride[k] % V != 0) al = false;
         }
         max_off = std::max(max_off, lmax);
         int64_t is = lv.stride[p.rank - 1];

@@ -84,7 +84,7 @@ constexpr int kMaxRank = XG_MAX_RANK;
 
 // How a leaf is read along the innermost iteration dimension.
 enum LeafMode : uint8_t {
-    LM_CONTIG = 0,  // inner stride 1 and vector-aligned: wide loads
+    LM_CONTIG = 0,  // inner stride 1, element-aligned: wide loads
     LM_BCAST = 1,   // inner stride 0: one load per chunk
     LM_STRIDED = 2, // anything else: one load per element
     LM_GATHER = 3,  // read at computed offsets (MO_GATHER); stride[0..1] = valid offset range
@@ -174,6 +174,7 @@ struct EwPlan {
     int32_t out_mode;        // LM_CONTIG or LM_STRIDED, | LM_NT, | LM_FILL
     int32_t index64;         // 1 if any offset needs 64-bit arithmetic
     uint32_t fill_zero;      // always 0: ties a granule-fill read into the stored value
+    uint32_t xcd_runs;       // 1: each XCD takes one contiguous run of the launch's workgroups
     int64_t shape[kMaxRank];
     FastDiv div[kMaxRank];   // div[k] divides by shape[k] (outer dims)
     uint32_t inner;          // shape[rank-1]
