@@ -232,3 +232,19 @@ def lib():
             f.argtypes = args
         _lib = L
     return _lib
+
+
+NATIVE_PATH = os.path.join(HERE, "lib", "_xgpy.so")
+
+
+def native():
+    """The compiled tree walker (cpp/pyeval.cpp) over libxg.so."""
+    lib()  # torch's HIP runtime first, then the library it links
+    if not os.path.exists(NATIVE_PATH):
+        raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+    import importlib.machinery
+    import importlib.util
+    loader = importlib.machinery.ExtensionFileLoader("_xgpy", NATIVE_PATH)
+    m = importlib.util.module_from_spec(importlib.util.spec_from_loader("_xgpy", loader))
+    loader.exec_module(m)
+    return m

@@ -19,6 +19,7 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -133,6 +134,16 @@ def build(force: bool = False, jobs: int | None = None) -> str:
         _run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include",
               "-I", INCLUDE, loop_src, "-o", loop_lib, "-L", LIBDIR, "-lxg", "-L", "/opt/rocm/lib", "-lamdhip64",
               "-Wl,-rpath,$ORIGIN", "-Wl,-rpath,/opt/rocm/lib"])
+
+    # 5. the front end's tree walker (a CPython extension over libxg.so)
+    py_src = os.path.join(HERE, "cpp", "pyeval.cpp")
+    py_lib = os.path.join(LIBDIR, "_xgpy.so")
+    if force or not os.path.exists(py_lib) or _newest([py_src, LIB] + headers) > os.path.getmtime(py_lib):
+        tmp = py_lib + ".tmp"
+        _run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-I", sysconfig.get_paths()["include"], "-I", INCLUDE,
+              py_src, "-o", tmp, "-L", LIBDIR, "-lxg", "-L", "/opt/rocm/lib", "-Wl,-rpath,$ORIGIN",
+              "-Wl,-rpath,/opt/rocm/lib"])
+        os.replace(tmp, py_lib)
     return LIB
 
 

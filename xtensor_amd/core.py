@@ -28,6 +28,7 @@ from __future__ import annotations
 
 import builtins
 import ctypes as C
+import math
 import numbers
 import os
 from typing import Any, Callable, Iterable, Sequence
@@ -99,37 +100,52 @@ def _check(status: int) -> None:
 
 # ----------------------------------------------------------------------------
 # expressions
+_NEGATE = A.OP["NEGATE"]
+
+
+def _operator(name):
+    """The methods of a binary operator: self op o, and o op self."""
+    code = A.OP[name]
+
+    def f(self, o):
+        n = Func.__new__(Func)
+        n.op = code
+        n.args = (self, o if isinstance(o, Expr) else Scalar(o))
+        n.index = 0
+        return n
+
+    def r(self, o):
+        n = Func.__new__(Func)
+        n.op = code
+        n.args = (o if isinstance(o, Expr) else Scalar(o), self)
+        n.index = 0
+        return n
+    return f, r
+
+
 class Expr:
     """A node of a lazy expression tree (xfunction / xscalar / container)."""
 
+    __slots__ = ()
+
     # ---- arithmetic operators (core/xoperation.hpp:231-545)
-    def __add__(self, o): return Func(A.OP["PLUS"], self, o)
-    def __radd__(self, o): return Func(A.OP["PLUS"], o, self)
-    def __sub__(self, o): return Func(A.OP["MINUS"], self, o)
-    def __rsub__(self, o): return Func(A.OP["MINUS"], o, self)
-    def __mul__(self, o): return Func(A.OP["MULTIPLIES"], self, o)
-    def __rmul__(self, o): return Func(A.OP["MULTIPLIES"], o, self)
-    def __truediv__(self, o): return Func(A.OP["DIVIDES"], self, o)
-    def __rtruediv__(self, o): return Func(A.OP["DIVIDES"], o, self)
-    def __mod__(self, o): return Func(A.OP["MODULUS"], self, o)
-    def __rmod__(self, o): return Func(A.OP["MODULUS"], o, self)
-    def __and__(self, o): return Func(A.OP["BITWISE_AND"], self, o)
-    def __rand__(self, o): return Func(A.OP["BITWISE_AND"], o, self)
-    def __or__(self, o): return Func(A.OP["BITWISE_OR"], self, o)
-    def __ror__(self, o): return Func(A.OP["BITWISE_OR"], o, self)
-    def __xor__(self, o): return Func(A.OP["BITWISE_XOR"], self, o)
-    def __rxor__(self, o): return Func(A.OP["BITWISE_XOR"], o, self)
-    def __lshift__(self, o): return Func(A.OP["LEFT_SHIFT"], self, o)
-    def __rlshift__(self, o): return Func(A.OP["LEFT_SHIFT"], o, self)
-    def __rshift__(self, o): return Func(A.OP["RIGHT_SHIFT"], self, o)
-    def __rrshift__(self, o): return Func(A.OP["RIGHT_SHIFT"], o, self)
-    def __neg__(self): return Func(A.OP["NEGATE"], self)
+    __add__, __radd__ = _operator("PLUS")
+    __sub__, __rsub__ = _operator("MINUS")
+    __mul__, __rmul__ = _operator("MULTIPLIES")
+    __truediv__, __rtruediv__ = _operator("DIVIDES")
+    __mod__, __rmod__ = _operator("MODULUS")
+    __and__, __rand__ = _operator("BITWISE_AND")
+    __or__, __ror__ = _operator("BITWISE_OR")
+    __xor__, __rxor__ = _operator("BITWISE_XOR")
+    __lshift__, __rlshift__ = _operator("LEFT_SHIFT")
+    __rshift__, __rrshift__ = _operator("RIGHT_SHIFT")
+    __lt__ = _operator("LESS")[0]
+    __le__ = _operator("LESS_EQUAL")[0]
+    __gt__ = _operator("GREATER")[0]
+    __ge__ = _operator("GREATER_EQUAL")[0]
+    def __neg__(self): return Func(_NEGATE, self)
     def __pos__(self): return Func(A.OP["IDENTITY"], self)
     def __invert__(self): return Func(A.OP["BITWISE_NOT"], self)
-    def __lt__(self, o): return Func(A.OP["LESS"], self, o)
-    def __le__(self, o): return Func(A.OP["LESS_EQUAL"], self, o)
-    def __gt__(self, o): return Func(A.OP["GREATER"], self, o)
-    def __ge__(self, o): return Func(A.OP["GREATER_EQUAL"], self, o)
     __hash__ = object.__hash__
 
     def equal(self, o):
@@ -162,6 +178,8 @@ class Expr:
 
 class Scalar(Expr):
     """xt::xscalar leaf: a value with a C++ type (containers/xscalar.hpp)."""
+
+    __slots__ = ("dtype_code", "value")
 
     def __init__(self, value, dtype=None):
         if dtype is None:
@@ -204,9 +222,11 @@ def _wrap(x) -> Expr:
 class Func(Expr):
     """xfunction node: functor `op` applied to argument expressions."""
 
+    __slots__ = ("op", "args", "index")
+
     def __init__(self, op: int, *args, index: int = 0):
         self.op = op
-        self.args = tuple(_wrap(a) for a in args)
+        self.args = tuple([a if isinstance(a, Expr) else Scalar(a) for a in args])
         self.index = index
 
 
@@ -296,11 +316,34 @@ class DeviceArray(Expr):
         return f"DeviceArray(shape={self._shape}, dtype={self.dtype}, strides={self.strides}, offset={self.offset})"
 
 
+def _array(storage, code: int, shape: tuple, strides: tuple, offset: int) -> DeviceArray:
+    """A DeviceArray of arguments that already have their final types."""
+    a = DeviceArray.__new__(DeviceArray)
+    a.storage = storage
+    a.dtype_code = code
+    a._shape = shape
+    a.strides = strides
+    a.offset = offset
+    return a
+
+
 def _row_major_strides(shape: Sequence[int]) -> tuple:
     st = [1] * len(shape)
     for k in range(len(shape) - 2, -1, -1):
         st[k] = st[k + 1] * max(int(shape[k + 1]), 1)
     return tuple(st)
+
+
+_torch_module = None
+
+
+def _torch():
+    """The torch module, imported on first use."""
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        _torch_module = torch
+    return _torch_module
 
 
 def _torch_device(device):
@@ -309,12 +352,15 @@ def _torch_device(device):
 
 def empty(shape, dtype="float64", device=None) -> DeviceArray:
     """Uninitialised device array (xt::xarray<T>::from_shape)."""
-    import torch
-    shape = tuple(int(s) for s in (shape if isinstance(shape, (tuple, list)) else (shape,)))
-    code = dtype_code(dtype)
-    n = int(np.prod(shape, dtype=np.int64)) if shape else 1
-    storage = torch.empty(max(n * A.DTYPE_SIZE[code], 1), dtype=torch.uint8, device=_torch_device(device))
-    return DeviceArray(storage, code, shape)
+    shape = tuple([int(s) for s in (shape if isinstance(shape, (tuple, list)) else (shape,))])
+    return _empty(shape, dtype_code(dtype), device)
+
+
+def _empty(shape: tuple, code: int, device=None) -> DeviceArray:
+    torch = _torch()
+    n = math.prod(shape) * A.DTYPE_SIZE[code]
+    storage = torch.empty(n if n > 0 else 1, dtype=torch.uint8, device=device or "cuda")
+    return _array(storage, code, shape, _row_major_strides(shape), 0)
 
 
 def zeros(shape, dtype="float64", device=None) -> DeviceArray:
@@ -376,17 +422,21 @@ def newaxis():
 def _norm_key(a: DeviceArray, keys) -> list:
     """Expand Ellipsis and pad with all() (xt::view keeps trailing dims)."""
     keys = list(keys)
-    n_ell = builtins.sum(1 for k in keys if k is Ellipsis)
-    if n_ell > 1:
-        raise IndexError("only one Ellipsis allowed")
-    consumed = builtins.sum(1 for k in keys if not isinstance(k, _NewAxis) and k is not None and k is not Ellipsis)
-    if consumed > a.ndim:
+    ell, consumed = -1, 0
+    for i, k in enumerate(keys):
+        if k is Ellipsis:
+            if ell >= 0:
+                raise IndexError("only one Ellipsis allowed")
+            ell = i
+        elif k is not None and type(k) is not _NewAxis:
+            consumed += 1
+    rest = len(a._shape) - consumed
+    if rest < 0:
         raise IndexError("too many indices")
-    if n_ell:
-        i = keys.index(Ellipsis)
-        keys[i:i + 1] = [_All()] * (a.ndim - consumed)
-    else:
-        keys += [_All()] * (a.ndim - consumed)
+    if ell >= 0:
+        keys[ell:ell + 1] = [_All()] * rest
+    elif rest:
+        keys += [_All()] * rest
     return keys
 
 
@@ -401,25 +451,25 @@ def view(a: DeviceArray, *keys) -> DeviceArray:
         raise TypeError("views are taken of device arrays")
     keys = _norm_key(a, keys)
     shape, strides = [], []
-    offset = a.offset
+    ashape, astrides, offset = a._shape, a.strides, a.offset
     dim = 0
     for k in keys:
-        if isinstance(k, _NewAxis) or k is None:
+        t = type(k)
+        if k is None or t is _NewAxis:
             shape.append(1)
             strides.append(0)
             continue
-        n, s = a.shape[dim], a.strides[dim]
-        if isinstance(k, _All):
+        n, s = ashape[dim], astrides[dim]
+        if t is _All:
             shape.append(n)
             strides.append(s)
-        elif isinstance(k, (slice, range_)):
-            sl = k.as_slice() if isinstance(k, range_) else k
-            start, stop, step = sl.indices(n)
-            cnt = len(range(start, stop, step))
+        elif t is slice or t is range_:
+            r = range(*(k if t is slice else k.as_slice()).indices(n))
+            cnt = len(r)
             if cnt > 0:
-                offset += start * s
+                offset += r.start * s
             shape.append(cnt)
-            strides.append(s * step)
+            strides.append(s * r.step)
         elif isinstance(k, (numbers.Integral, np.integer)):
             i = int(k)
             if i < 0:
@@ -430,7 +480,7 @@ def view(a: DeviceArray, *keys) -> DeviceArray:
         else:
             raise TypeError(f"unsupported view key {k!r}")
         dim += 1
-    return DeviceArray(a.storage, a.dtype_code, shape, strides, offset)
+    return _array(a.storage, a.dtype_code, tuple(shape), tuple(strides), offset)
 
 
 strided_view = view
@@ -442,7 +492,8 @@ def transpose(a: DeviceArray, perm: Sequence[int] | None = None) -> DeviceArray:
         perm = list(range(a.ndim))[::-1]
     if sorted(perm) != list(range(a.ndim)):
         raise RuntimeError("transpose: permutation is not a permutation of the axes")
-    return DeviceArray(a.storage, a.dtype_code, [a.shape[p] for p in perm], [a.strides[p] for p in perm], a.offset)
+    return _array(a.storage, a.dtype_code, tuple([a._shape[p] for p in perm]), tuple([a.strides[p] for p in perm]),
+                  a.offset)
 
 
 def broadcast(a, shape: Sequence[int]):
@@ -524,6 +575,7 @@ class Reducer(Expr):
     def __init__(self, kind, e, axes=None, keep_dims=False, initial=None, dtype=None, ddof=0,
                  evaluation_strategy="lazy"):
         self.kind = kind
+        self.op = A.RED[kind]
         self.ddof = int(ddof)
         if evaluation_strategy not in ("lazy", "immediate"):
             raise ValueError("evaluation_strategy is 'lazy' or 'immediate'")
@@ -540,7 +592,7 @@ class Reducer(Expr):
 
     def to_abi(self) -> A.ReduceDesc:
         d = A.ReduceDesc()
-        d.op = A.RED[self.kind]
+        d.op = self.op
         d.acc_dtype = self.acc_dtype
         if self.axes is None:
             d.n_axes = -1
@@ -682,13 +734,16 @@ def _shape_of(ndim, shp):
     return tuple(int(shp[i]) for i in range(ndim))
 
 
+def _info(r):
+    """(dtype code, shape) from a Packed info call, or the status it returned."""
+    if type(r) is int:
+        _check(r)
+    return r
+
+
 def expr_info(e: Expr):
     """(dtype code, broadcast shape) of an expression, from the library."""
-    s = serialize(e, reducer_fn=lambda r: _placeholder_for(r))
-    dt, nd = C.c_int32(), C.c_int32()
-    shp = (C.c_int64 * A.MAX_RANK)()
-    _check(A.lib().xg_expr_info(s.ptr(), C.byref(dt), C.byref(nd), shp))
-    return dt.value, _shape_of(nd.value, shp)
+    return _info(_pack(e, _placeholder_for).info())
 
 
 class _Placeholder(DeviceArray):
@@ -708,19 +763,34 @@ def _placeholder_for(r: Reducer):
 
 
 def reduce_info(r: Reducer):
-    s = serialize(r.expr, reducer_fn=lambda x: _placeholder_for(x))
-    d = r.to_abi()
-    dt, nd = C.c_int32(), C.c_int32()
-    shp = (C.c_int64 * A.MAX_RANK)()
-    _check(A.lib().xg_reduce_info(s.ptr(), C.byref(d), C.byref(dt), C.byref(nd), shp))
-    return dt.value, _shape_of(nd.value, shp)
+    return _info(_pack(r.expr, _placeholder_for).reduce_info(r))
+
+
+_native = None
+
+
+def _pack(e: Expr, reducer_fn):
+    """The tree of e as a descriptor of the C ABI, with the library's calls on
+    it as methods (cpp/pyeval.cpp); reducers inside it are evaluated first, by
+    reducer_fn."""
+    global _native
+    if _native is None:
+        m = A.native()
+        m.setup((DeviceArray, _Placeholder, Func, Scalar, Reducer, IndexView))
+        _native = m
+    return _native.pack(e, reducer_fn)
 
 
 # ----------------------------------------------------------------------------
 # evaluation
 def _stream():
-    import torch
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(_raw_stream())
+
+
+def _raw_stream() -> int:
+    """The address of torch's current stream on the current device."""
+    c = _torch()._C
+    return c._cuda_getCurrentRawStream(c._cuda_getDevice())
 
 
 def _require_device(arrs: Iterable[DeviceArray]):
@@ -748,18 +818,19 @@ def _leaves(e) -> list:
 
 
 def _eval_reducer(r: Reducer) -> DeviceArray:
-    dt, shp = reduce_info(r)
-    out = empty(shp, dt)
-    _reduce_into(r, out)
+    p = _pack(r.expr, _eval_reducer)
+    dt, shp = _info(p.reduce_info(r))
+    out = _empty(shp, dt)
+    st = p.reduce(r, out, _raw_stream())
+    if st:
+        _check(st)
     return out
 
 
 def _reduce_into(r: Reducer, out: DeviceArray) -> None:
-    _require_device(_leaves(r.expr) + [out])
-    s = serialize(r.expr, reducer_fn=_eval_reducer)
-    d = r.to_abi()
-    t = out.to_abi()
-    _check(A.lib().xg_reduce(s.ptr(), C.byref(d), C.byref(t), _stream()))
+    st = _pack(r.expr, _eval_reducer).reduce(r, out, _raw_stream())
+    if st:
+        _check(st)
 
 
 def assign(out, e):
@@ -770,10 +841,9 @@ def assign(out, e):
     if isinstance(e, Reducer):
         _reduce_into(e, out)
         return out
-    _require_device(_leaves(e) + [out])
-    s = serialize(e, reducer_fn=_eval_reducer)
-    t = out.to_abi()
-    _check(A.lib().xg_assign(s.ptr(), C.byref(t), _stream()))
+    st = _pack(e, _eval_reducer).assign(out, _raw_stream())
+    if st:
+        _check(st)
     return out
 
 
@@ -865,9 +935,13 @@ def eval(e) -> DeviceArray:  # noqa: A001
         return e  # already a row-major container
     if isinstance(e, Reducer):
         return _eval_reducer(e)
-    dt, shp = expr_info(e)
-    out = empty(shp, dt)
-    return assign(out, e)
+    p = _pack(e, _eval_reducer)
+    dt, shp = _info(p.info())
+    out = _empty(shp, dt)
+    st = p.assign(out, _raw_stream())
+    if st:
+        _check(st)
+    return out
 
 
 # ----------------------------------------------------------------------------
@@ -1095,18 +1169,15 @@ class Scan:
 
 def _scan(kind, e, axis=None, dtype=None) -> DeviceArray:
     e = _wrap(e)
-    d = A.ScanDesc()
-    d.op = A.SCAN[kind]
-    d.acc_dtype = -1 if dtype is None else dtype_code(dtype)
-    d.axis = A.AXIS_NONE if axis is None else int(axis)
-    s = serialize(e, reducer_fn=_eval_reducer)
-    dt, nd = C.c_int32(), C.c_int32()
-    shp = (C.c_int64 * A.MAX_RANK)()
-    _check(A.lib().xg_scan_info(s.ptr(), C.byref(d), C.byref(dt), C.byref(nd), shp))
-    out = empty(_shape_of(nd.value, shp), dt.value)
-    _require_device(_leaves(e) + [out])
-    t = out.to_abi()
-    _check(A.lib().xg_scan(s.ptr(), C.byref(d), C.byref(t), _stream()))
+    op = A.SCAN[kind]
+    acc = -1 if dtype is None else dtype_code(dtype)
+    ax = A.AXIS_NONE if axis is None else int(axis)
+    p = _pack(e, _eval_reducer)
+    dt, shp = _info(p.scan_info(op, acc, ax))
+    out = _empty(shp, dt)
+    st = p.scan(op, acc, ax, out, _raw_stream())
+    if st:
+        _check(st)
     return out
 
 

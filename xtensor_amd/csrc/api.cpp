@@ -693,6 +693,32 @@ void reduce_top(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out,
 void xg::reduce_call(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out, hipStream_t st, BlockSource src,
                      void* ctx, bool counters) {
     const char* used = nullptr;
+    // one plan and at most one block (its split partials): planned once
+    const bool lone = e && r && !(r->flags & ~XG_REDUCE_IMMEDIATE) &&
+                      (!(r->flags & XG_REDUCE_IMMEDIATE) ||
+                       (e->n_nodes == 1 && e->nodes && e->nodes[0].op == XG_OP_LEAF)) &&
+                      r->op != XG_RED_VARIANCE && r->op != XG_RED_STDDEV && r->op != XG_RED_MINMAX;
+    if (lone) {
+        int V = 4;
+        RedPlan p{};
+        bool whole = true;
+        try {
+            p = plan_reduce_best(e, r, out, &V);
+        } catch (const Error& err) {
+            if (err.code != XG_UNSUPPORTED) throw;
+            whole = false;  // in pieces, or refused, below
+        }
+        if (whole) {
+            if (p.n_out) {
+                const size_t bytes = reduce_workspace_bytes(p);
+                p.partials = bytes ? src(bytes, st, ctx) : nullptr;
+                p.counters = counters ? reduce_counters(st) : nullptr;
+                check_hip(launch_reduce(p, V, st, &used), "reduction launch");
+            }
+            note_kernel(used ? used : "empty");
+            return;
+        }
+    }
     Arena sizing;
     reduce_top(e, r, out, st, sizing, &used);
     Arena a;

@@ -21,6 +21,7 @@
 #include <map>
 #include <mutex>
 #include <sstream>
+#include <unordered_map>
 #include <vector>
 
 #include "spec_emit.hpp"
@@ -43,6 +44,10 @@ struct Entry {
     JitKernel k;
 };
 std::map<std::string, Entry> g_entries;  // key: device | name expression | source
+// the loaded kernels by the bytes that determine their source (see key_of):
+// writing the source out to look a kernel up took most of a launch's host time
+// (a fused float64 sum of [4096, 2048] 70 us of GPU time in 138 us a pair)
+std::unordered_map<std::string, const JitKernel*> g_loaded;
 
 struct Env {
     bool ok = false;
@@ -283,16 +288,64 @@ bool jit_wanted(uint64_t elements) {
     return m == 2 || (m == 1 && elements >= g_min_elements);
 }
 
+namespace {
+
+// Everything the text of a specialisation depends on (spec_emit.hpp): the
+// device, the kernel and its template arguments (`head`), and the program with
+// its leaves' types and access modes.
+std::string key_of(std::initializer_list<int> head, const Program& prog, const LeafView* leaves) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return {};
+    std::string k;
+    k.reserve(head.size() * 4 + size_t(prog.nops) * sizeof(MicroOp) + size_t(prog.nleaves) * 2 + 20);
+    auto put = [&](int v) { k.append(reinterpret_cast<const char*>(&v), sizeof v); };
+    put(dev);
+    for (int v : head) put(v);
+    put(prog.nops);
+    put(prog.nregs);
+    put(prog.nleaves);
+    put(prog.result_reg);
+    k.append(reinterpret_cast<const char*>(prog.ops), size_t(prog.nops) * sizeof(MicroOp));
+    for (int l = 0; l < prog.nleaves; ++l) {
+        k.push_back(char(leaves[l].dtype));
+        k.push_back(char(lm_base(leaves[l].mode)));
+    }
+    return k;
+}
+
+const JitKernel* find_loaded(const std::string& key) {
+    if (key.empty()) return nullptr;
+    std::lock_guard<std::mutex> lk(g_mu);
+    const auto f = g_loaded.find(key);
+    if (f == g_loaded.end()) return nullptr;
+    ++g_stats.memory_hits;
+    return f->second;
+}
+
+const JitKernel* remember(const std::string& key, const JitKernel* k) {
+    if (k && !key.empty()) {
+        std::lock_guard<std::mutex> lk(g_mu);
+        g_loaded.emplace(key, k);
+    }
+    return k;
+}
+
+}  // namespace
+
 const JitKernel* jit_ew(const EwPlan& p, int V) {
     if (!p.compact || p.rank < 1 || p.rank > 4) return nullptr;
+    const std::string key = key_of({0, V, p.rank, p.out_dtype, lm_base(p.out_mode)}, p.prog, p.leaves);
+    if (const JitKernel* k = find_loaded(key)) return k;
     const std::string src = "#include \"ew_kernels.hpp\"\n" + emit_ew_spec("JitSpec", p, V);
     const std::string expr = "&xg::ew_spec_kernel<" + std::to_string(V) + ", " + std::to_string(p.prog.nregs) +
                              ", JitSpec, " + std::to_string(p.rank) + ">";
-    return get(src, expr);
+    return remember(key, get(src, expr));
 }
 
 const JitKernel* jit_reduce(const RedPlan& p, int V, int kind) {
     if (p.index64) return nullptr;
+    const std::string key = key_of({1 + kind, V, p.acc, p.op}, p.prog, p.leaves);
+    if (const JitKernel* k = find_loaded(key)) return k;
     const std::string src = "#include \"reduce_kernels.hpp\"\n" + emit_red_spec("JitSpec", p, V);
     const std::string head = std::to_string(V) + ", " + std::to_string(p.prog.nregs) + ", JitSpec, ";
     const std::string ao = std::to_string(p.acc) + ", " + std::to_string(p.op);
@@ -305,7 +358,7 @@ const JitKernel* jit_reduce(const RedPlan& p, int V, int kind) {
     case JR_COLS: expr = "&xg::reduce_cols_kernel<" + head + "false, " + ao + ", 4>"; break;
     default: return nullptr;
     }
-    return get(src, expr);
+    return remember(key, get(src, expr));
 }
 
 const JitKernel* jit_assign_rc(const EwPlan& p, int V, int rak, int rop, int cak, int cop, int ul) {
