@@ -30,6 +30,14 @@ hipError_t launch_scan(const ScanPlan& p, int V, void* ws, hipStream_t stream, c
     ScanKernels k{};
     if (!scan_kernels_float(p.acc, p.op, &k) && !scan_kernels_int(p.acc, p.op, &k)) return hipErrorInvalidValue;
     dim3 block(256);
+    if (p.tiled == ST_SHORT) {
+        TFn f = k.shorts[p.tile_native ? 1 : 0];
+        const uint64_t columns = uint64_t(p.tile.outer) * p.tile.inner;
+        if (!f || columns >= (uint64_t(1) << 31)) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(f, dim3(uint32_t((columns + 255) / 256)), block, 0, stream, p.tile);
+        if (used) *used = "scan_short";
+        return hipGetLastError();
+    }
     if (p.tiled != ST_NONE) {
         const bool trans = p.tiled == ST_TRANS;
         TFn scan = k.tiles[p.tile_native ? 1 : 0][trans ? 1 : 0];
@@ -39,7 +47,9 @@ hipError_t launch_scan(const ScanPlan& p, int V, void* ws, hipStream_t stream, c
         if (t.nchunks > 1 && !ws) return hipErrorInvalidValue;
         if (t.single) {  // one pass: chunks of kTileLbRows rows and a look-back per column
             TFn one = k.tiles1p[p.tile_native ? 1 : 0][trans ? 1 : 0];
-            if (!one || t.chunk_rows != kTileLbRows) return hipErrorInvalidValue;
+            if (!one || t.lanes < 4 || t.lanes > 64 || (t.lanes & (t.lanes - 1)) || t.chunk_rows * t.lanes != kTileLbRows * 64u ||
+                (trans && t.lanes != 64))
+                return hipErrorInvalidValue;
             const uint64_t total = uint64_t(t.outer) * t.nchunks * t.ntiles;
             if (t.classes < 1 || t.classes > kTileMaxClasses || (uint64_t(t.outer) * t.ntiles) % t.classes)
                 return hipErrorInvalidValue;
@@ -51,7 +61,7 @@ hipError_t launch_scan(const ScanPlan& p, int V, void* ws, hipStream_t stream, c
             uint64_t n2;  // 16-byte words the init kernel clears: the packed words, or the flags
             if (t.packed) {
                 t.words = reinterpret_cast<uint64_t*>(w);
-                n2 = n / 2;  // ncols: a multiple of 128
+                n2 = n / 2;  // ncols: a multiple of 16
             } else {
                 const uint64_t nf = uint64_t(t.outer) * t.nchunks * t.ntiles;
                 t.flags = reinterpret_cast<uint32_t*>(w);

@@ -20,7 +20,8 @@ enum ScanLayout : int32_t {
 enum ScanTiled : int32_t {
     ST_NONE = 0,
     ST_COLS = 1,   // output contiguous along inner as well (cumsum(X, 0))
-    ST_TRANS = 2   // output contiguous along len (cumsum(transpose(X), 1))
+    ST_TRANS = 2,  // output contiguous along len (cumsum(transpose(X), 1))
+    ST_SHORT = 3   // as ST_COLS over a short axis: a thread per column
 };
 
 // Kernel argument of the tiled scans (pointers filled in at launch).
@@ -29,7 +30,7 @@ struct TileScan {
     char* out;
     Store* part;          // [outer][nchunks][ncols] chunk totals, then carries
     uint32_t outer, len, inner;
-    uint32_t nchunks, ntiles, chunk_rows, ncols;  // ncols = ntiles * 64 * V
+    uint32_t nchunks, ntiles, chunk_rows, ncols;  // ncols = ntiles * 64 * V (one pass: ntiles * lanes * V)
     int64_t in_s_outer, in_s_len;                 // elements; inner stride 1
     int64_t out_s_outer, out_s_len, out_s_inner;  // elements
     uint64_t identity;
@@ -46,10 +47,14 @@ struct TileScan {
     Store* agg;           // ... [outer][nchunks][ncols] column totals
     Store* pre;           // ... and inclusive prefixes
     int32_t packed;       // 1: `words`; 0: `flags`, `agg`, `pre`
+    uint32_t lanes;       // one pass: lanes of a wave per row (a power of two, 4 .. 64)
 };
 
-// Rows of one chunk of the one-pass tiled scan (held in registers whole).
+// Rows of one chunk of the one-pass tiled scan (held in registers whole) with
+// 64 lanes a row; 64 / lanes times that with fewer.
 constexpr uint32_t kTileLbRows = 64;
+// Rows that are not whole aligned vectors take ST_SHORT up to this axis length.
+constexpr uint32_t kShortAxis = 128;
 // its ticket counters (at most kTileMaxClasses, 256 bytes apart) and timeout
 // count at the head of the workspace
 constexpr uint32_t kTileMaxClasses = 16;
@@ -122,8 +127,8 @@ void set_scan_flat_single_pass(int on);
 
 // The direct rows kernels apply: rank <= 2 rows layout with 32-bit offsets,
 // a program that is one load of a leaf of the accumulation input type, the
-// leaf and the output contiguous along the axis, rows starting 16-byte
-// aligned, output elements of the same size, not bf16.
+// leaf and the output contiguous along the axis (at any element address),
+// output elements of the same size, not bf16.
 bool scan_direct_ok(const ScanPlan& p);
 
 // Result dtype / shape of a scan.

@@ -362,6 +362,7 @@ struct ScanKernels {
     SFn rows32, rows64, cols32, cols64;
     SFn direct[2][2];   // [native][waves per row: 1, 4]
     uint32_t wave_tile;  // elements of one wave's tile in the direct kernels
+    TFn shorts[2];       // [native]
     TFn tile_totals, tile_carry;
     TFn tiles[2][2];     // [native][transposed output]; the transposed one is native only
     TFn tiles1p[2][2];   // the one-pass form, likewise
@@ -378,6 +379,7 @@ template <int AK, int OP> ScanKernels scan_kernels() {
                        {{scan_rows_direct_kernel<AK, OP, false, 1>, scan_rows_direct_kernel<AK, OP, false, 4>},
                         {scan_rows_direct_kernel<AK, OP, true, 1>, scan_rows_direct_kernel<AK, OP, true, 4>}},
                        scan_wave_tile<typename ScanIn<AK>::T>(),
+                       {scan_short_kernel<AK, OP, false>, scan_short_kernel<AK, OP, true>},
                        scan_tiles_totals_kernel<AK, OP>,
                        scan_tiles_carry_kernel<AK, OP>,
                        {{scan_tiles_kernel<AK, OP, false, false>, nullptr},

@@ -78,9 +78,11 @@ int scan_in_dtype(int acc) {
 
 // The tiled scans (scan_tiled.hpp) apply when the program is one load of a
 // leaf of the accumulation input type, the leaf is contiguous along a dim
-// other than the scan axis with 16-byte aligned rows, and the output is
-// contiguous along that dim (ST_COLS) or along the scan axis (ST_TRANS);
-// outputs of another element size or bf16 keep the other kernels.
+// other than the scan axis, and the output is contiguous along that dim
+// (ST_COLS) or along the scan axis (ST_TRANS); outputs of another element size
+// or bf16 keep the other kernels.  Rows may start at any element address: the
+// scan_cols kernel, a thread walking the whole axis, took 72 ms on the columns
+// of an int32 [20510, 818] for a pitch that is no multiple of 16 bytes.
 void plan_tiled(ScanPlan* pp, int cus) {
     ScanPlan& p = *pp;
     p.tiled = ST_NONE;
@@ -91,7 +93,7 @@ void plan_tiled(ScanPlan* pp, int cus) {
     const int esz = dtype_size(in_dt);
     const int64_t V = 16 / esz;
     if (l.dtype != in_dt || p.out_dtype == XG_BFLOAT16 || dtype_size(p.out_dtype) != esz) return;
-    if (reinterpret_cast<uintptr_t>(l.ptr) % 16 || reinterpret_cast<uintptr_t>(p.out_ptr) % 16) return;
+    if (reinterpret_cast<uintptr_t>(l.ptr) % uintptr_t(esz) || reinterpret_cast<uintptr_t>(p.out_ptr) % uintptr_t(esz)) return;
     const bool native = p.out_dtype == in_dt && p.rdt == in_dt;
     TileScan t{};
     int kind = ST_NONE;
@@ -106,7 +108,6 @@ void plan_tiled(ScanPlan* pp, int cus) {
         t.out_s_outer = R == 3 ? p.out_stride[0] : 0;
         t.out_s_len = p.out_stride[R - 2];
         t.out_s_inner = 1;
-        if (t.out_s_outer % V || t.out_s_len % V) return;
         kind = ST_COLS;
     } else if (p.layout == SL_ROWS && (R == 2 || R == 3) && native) {
         if (l.stride[R - 2] != 1 || l.stride[R - 1] == 1 || p.out_stride[R - 1] != 1) return;
@@ -118,12 +119,21 @@ void plan_tiled(ScanPlan* pp, int cus) {
         t.out_s_outer = R == 3 ? p.out_stride[0] : 0;
         t.out_s_len = 1;
         t.out_s_inner = p.out_stride[R - 2];
-        if (t.out_s_outer % V || t.out_s_inner % V) return;
         kind = ST_TRANS;
     } else {
         return;
     }
-    if (t.in_s_outer % V || t.in_s_len % V || t.in_s_len < 0 || t.in_s_outer < 0) return;
+    if (t.in_s_len < 0 || t.in_s_outer < 0) return;
+    // Over a short axis, rows that are not whole aligned vectors take a thread
+    // per column (ST_SHORT): no chunks to connect, and neighbouring threads
+    // read neighbouring elements whatever the pitch.
+    const bool aligned = reinterpret_cast<uintptr_t>(l.ptr) % 16 == 0 && reinterpret_cast<uintptr_t>(p.out_ptr) % 16 == 0 &&
+                         t.in_s_outer % V == 0 && t.in_s_len % V == 0 && t.out_s_outer % V == 0 &&
+                         (kind == ST_COLS ? t.out_s_len : t.out_s_inner) % V == 0;
+    if (!aligned && t.len <= kShortAxis) {
+        if (kind != ST_COLS || uint64_t(t.outer) * t.inner >= (uint64_t(1) << 31)) return;
+        kind = ST_SHORT;
+    }
     const uint32_t sub = 64u;  // rows of one sub-tile (scan_tiles_kernel)
     const uint64_t cols = uint64_t(64 * V);
     t.ntiles = uint32_t((t.inner + cols - 1) / cols);
@@ -138,6 +148,7 @@ void plan_tiled(ScanPlan* pp, int cus) {
     t.chunk_rows = uint32_t((rows + sub - 1) / sub * sub);
     t.nchunks = uint32_t((uint64_t(t.len) + t.chunk_rows - 1) / t.chunk_rows);
     if (per_chunk * t.nchunks >= (uint64_t(1) << 31)) return;
+    if (kind == ST_SHORT) t.nchunks = 1;
     // One pass with a look-back per column when there are at least two
     // chunks.  Measured on MI355X faster than the three launches from one
     // column tile up (float32 cumsum along axis 0: [131072, 256] 99 against
@@ -145,14 +156,26 @@ void plan_tiled(ScanPlan* pp, int cus) {
     // 32-bit accumulators publish packed with their flag, 64-bit ones as
     // value, wait, flag per (chunk, tile).
     const bool packed = p.acc == AK_F32C || p.acc == AK_F32 || p.acc == AK_I32 || p.acc == AK_U32;
-    const uint64_t chunks1 = (uint64_t(t.len) + kTileLbRows - 1) / kTileLbRows;
-    if (g_tile_single_pass && chunks1 >= 2 && per_chunk * chunks1 < (uint64_t(1) << 31)) {
+    // rows narrower than a wave: fewer lanes a row and more rows a chunk, as
+    // long as two chunks remain
+    uint32_t lanes = 64;
+    if (kind == ST_COLS)
+        while (lanes > 4 && uint64_t(lanes / 2) * uint64_t(V) >= t.inner && uint64_t(t.len) * (lanes / 2) > kTileLbRows * 64u)
+            lanes /= 2;
+    const uint64_t rows1 = uint64_t(kTileLbRows) * (64u / lanes);
+    const uint64_t chunks1 = (uint64_t(t.len) + rows1 - 1) / rows1;
+    const uint64_t tiles1 = (t.inner + uint64_t(lanes) * V - 1) / (uint64_t(lanes) * V);
+    const uint64_t chains = uint64_t(t.outer) * tiles1;
+    if (kind != ST_SHORT && g_tile_single_pass && chunks1 >= 2 && chains * chunks1 < (uint64_t(1) << 31)) {
         t.packed = packed ? 1 : 0;
         t.single = 1;
-        t.chunk_rows = kTileLbRows;
+        t.lanes = lanes;
+        t.ntiles = uint32_t(tiles1);
+        t.ncols = uint32_t(tiles1 * lanes * uint64_t(V));
+        t.chunk_rows = uint32_t(rows1);
         t.nchunks = uint32_t(chunks1);
         t.classes = 1;  // the largest power of two up to kTileMaxClasses dividing the chains
-        while (t.classes < kTileMaxClasses && per_chunk % (2 * t.classes) == 0) t.classes *= 2;
+        while (t.classes < kTileMaxClasses && chains % (2 * t.classes) == 0) t.classes *= 2;
     }
     t.in = l.ptr;
     t.out = p.out_ptr;
@@ -217,9 +240,7 @@ bool scan_direct_ok(const ScanPlan& p) {
     const int esz = dtype_size(l.dtype);
     if (l.dtype != scan_in_dtype(p.acc) || lm_base(l.mode) != LM_CONTIG || l.stride[p.rank - 1] != 1) return false;
     if (p.out_dtype == XG_BFLOAT16 || dtype_size(p.out_dtype) != esz || p.out_stride[p.rank - 1] != 1) return false;
-    if (reinterpret_cast<uintptr_t>(l.ptr) % 16 || reinterpret_cast<uintptr_t>(p.out_ptr) % 16) return false;
-    if (p.rank == 2 && ((l.stride[0] * esz) % 16 || (p.out_stride[0] * esz) % 16)) return false;
-    return true;
+    return reinterpret_cast<uintptr_t>(l.ptr) % uintptr_t(esz) == 0 && reinterpret_cast<uintptr_t>(p.out_ptr) % uintptr_t(esz) == 0;
 }
 
 size_t scan_workspace_bytes(const ScanPlan& p) {
@@ -329,15 +350,18 @@ ScanPlan plan_scan(const xg_expr* e, const xg_scan_desc* s, const xg_tensor* out
         p.rows = uint32_t(outer * p.nchunks_in);
     }
     if (outer >= (uint64_t(1) << 31)) raise(XG_UNSUPPORTED, "scan too large for 32-bit indexing");
-    // out vector stores along the last dim when contiguous and aligned
-    bool oal = p.out_stride[p.rank - 1] == 1 && reinterpret_cast<uintptr_t>(p.out_ptr) % uintptr_t(osz * V) == 0;
-    for (int k = 0; k + 1 < p.rank; ++k)
-        if (p.out_stride[k] % V != 0) oal = false;
-    p.out_mode = oal ? LM_CONTIG : LM_STRIDED;
+    // out vector stores along the last dim when contiguous; non-temporal ones
+    // only for rows that start on 16-byte boundaries (see plan_assign)
+    p.out_mode = p.out_stride[p.rank - 1] == 1 && reinterpret_cast<uintptr_t>(p.out_ptr) % uintptr_t(osz) == 0 ? LM_CONTIG
+                                                                                                             : LM_STRIDED;
     {
         int64_t total = 1;
-        for (int k = 0; k < p.rank; ++k) total *= std::max<int64_t>(p.shape[k], 0);
-        if (total * osz >= kNtMinBytes) p.out_mode |= LM_NT;
+        bool rows16 = reinterpret_cast<uintptr_t>(p.out_ptr) % 16 == 0;
+        for (int k = 0; k < p.rank; ++k) {
+            total *= std::max<int64_t>(p.shape[k], 0);
+            if (p.out_stride[k] != 1) rows16 = rows16 && (p.out_stride[k] * osz) % 16 == 0;
+        }
+        if (rows16 && total * osz >= kNtMinBytes) p.out_mode |= LM_NT;
     }
     for (int pl = 0; pl < nl; ++pl) {
         LeafView& lv = p.leaves[pl];
@@ -349,12 +373,11 @@ ScanPlan plan_scan(const xg_expr* e, const xg_scan_desc* s, const xg_tensor* out
         int esz = dtype_size(t.dtype);
         lv.ptr = static_cast<const char*>(t.data) + t.offset * esz;
         lv.dtype = t.dtype;
-        bool al = reinterpret_cast<uintptr_t>(lv.ptr) % uintptr_t(esz * V) == 0;
+        const bool al = reinterpret_cast<uintptr_t>(lv.ptr) % uintptr_t(esz) == 0;
         int64_t lmax = 0;
         for (int k = 0; k < p.rank; ++k) {
             lv.stride[k] = order[size_t(k)].leaf[pl];
             lmax += (order[size_t(k)].n - 1) * std::abs(lv.stride[k]);
-            if (k + 1 < p.rank && lv.stride[k] % V != 0) al = false;
         }
         max_off = std::max(max_off, lmax);
         int64_t is = lv.stride[p.rank - 1];

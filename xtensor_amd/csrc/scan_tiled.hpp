@@ -33,7 +33,7 @@
 
 namespace xg {
 
-// V elements of type T (16 bytes, aligned) from ptr
+// V elements of type T (16 bytes) from ptr, at any element address
 template <int V, bool NT, class T> __device__ __forceinline__ void load_row(const T* ptr, T (&x)[V]) {
     Reg q[V];
     load_vec<V, NT>(reinterpret_cast<const char*>(ptr), int(sizeof(T)), ScanInDtype<T>::value, q);
@@ -45,6 +45,59 @@ template <int V, bool NT, class T> __device__ __forceinline__ void load_row(cons
 template <int V, class T> __device__ __forceinline__ void load_row_partial(const T* ptr, bool ok, int nv, T (&x)[V]) {
 #pragma unroll
     for (int v = 0; v < V; ++v) x[v] = (ok && v < nv) ? ptr[v] : T(0);
+}
+
+// N rows of a lane's columns in a tile that ends inside the row: rows row0 +
+// i * step, those past the chunk clamped to its last one.  Lanes with all V
+// columns take whole vectors, the lane the row ends in its columns one by one,
+// lanes past it nothing; one branch around all rows' loads, so that they issue
+// together (a branch per row made each wait for the one before).
+template <int N, int V, class T>
+__device__ __forceinline__ void load_rows_edge(const T* base, int64_t s_len, uint32_t row0, uint32_t step, uint32_t r1,
+                                               int nv, T (&x)[N][V]) {
+    if (nv == V) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            load_row<V, false>(base + int64_t(min(row0 + uint32_t(i) * step, r1 - 1)) * s_len, x[i]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const uint32_t row = row0 + uint32_t(i) * step;
+            load_row_partial<V>(base + int64_t(min(row, r1 - 1)) * s_len, row < r1, nv, x[i]);
+        }
+    }
+}
+
+// A short axis (at most kShortAxis rows), any pitch: a thread per column walks
+// its rows, 16 of them in flight.  Bound by the latency of len / 16 rounds of
+// loads (float32 [100, 12001]: 18.9 us a call).
+template <int AK, int OP, bool NATIVE>
+__global__ __launch_bounds__(256) void scan_short_kernel(const TileScan p) {
+    using A = Acc<AK, OP>;
+    using T = typename ScanIn<AK>::T;
+    constexpr int U = 16;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= p.outer * p.inner) return;
+    const uint32_t o = i / p.inner, col = i - o * p.inner;
+    const T* in = reinterpret_cast<const T*>(p.in) + int64_t(o) * p.in_s_outer + col;
+    const int odt = NATIVE ? int(ScanInDtype<T>::value) : p.out_dtype;
+    const int rdt = NATIVE ? int(ScanInDtype<T>::value) : p.rdt;
+    const int oesz = dtype_size(odt);
+    char* out = p.out + (int64_t(o) * p.out_s_outer + col) * oesz;
+    A run;
+    run.init(p.identity);
+    for (uint32_t r = 0; r < p.len; r += U) {
+        T x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = in[int64_t(min(r + uint32_t(u), p.len - 1)) * p.in_s_len];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (r + uint32_t(u) >= p.len) break;  // uniform
+            run.add(reg_put<T>(x[u]));
+            const Reg val = run.value(rdt);
+            store_raw(out + int64_t(r + uint32_t(u)) * p.out_s_len * oesz, oesz, NATIVE ? val : cvt(val, rdt, odt));
+        }
+    }
 }
 
 template <int AK, int OP>
@@ -82,11 +135,7 @@ __global__ __launch_bounds__(256) void scan_tiles_totals_kernel(const TileScan p
             for (int u = 0; u < U; ++u)
                 load_row<V, false>(base + int64_t(min(r + 4u * uint32_t(u), r1 - 1)) * p.in_s_len, x[u]);
         } else {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t row = r + 4u * uint32_t(u);
-                load_row_partial<V>(base + int64_t(min(row, r1 - 1)) * p.in_s_len, row < r1, nv, x[u]);
-            }
+            load_rows_edge<U, V>(base, p.in_s_len, r, 4u, r1, nv, x);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -213,11 +262,7 @@ __global__ __launch_bounds__(256) void scan_tiles_kernel(const TileScan p) {
             for (int i = 0; i < RW; ++i)
                 load_row<V, false>(base + int64_t(min(rw0 + uint32_t(i), r1 - 1)) * p.in_s_len, x[i]);
         } else {
-#pragma unroll
-            for (int i = 0; i < RW; ++i) {
-                const uint32_t row = rw0 + uint32_t(i);
-                load_row_partial<V>(base + int64_t(min(row, r1 - 1)) * p.in_s_len, row < r1, nv, x[i]);
-            }
+            load_rows_edge<RW, V>(base, p.in_s_len, rw0, 1u, r1, nv, x);
         }
         // this wave's totals, then the prefix of the waves before it
         A pre[V];

@@ -23,6 +23,11 @@
 //     inclusive prefix;
 //   * the chunk is scanned from those prefixes and stored, as in the scan
 //     phase of the three-launch form.
+// A row of fewer than 64 vectors does not fill a wave: then `lanes` = L lanes
+// take a row, a wave holds 64 / L groups of 16 rows below each other, and a
+// chunk has 64 * 64 / L rows, so a narrow matrix has fewer, larger chunks and
+// whole waves (int64 [16054, 25] down the columns 26.5 us; the scan_cols kernel
+// that such odd pitches fell to took about 47 ms).
 // Publications of 32-bit accumulators (float32 sums with compensation,
 // float32 products, 32-bit integers) are one 64-bit word per (chunk, column)
 // holding the value and its flag (the packed form of scan_lookback.hpp),
@@ -207,17 +212,14 @@ __global__ __launch_bounds__(256) void scan_tiles_1p_kernel(const TileScan p) {
     constexpr int V = int(16 / sizeof(T));
     constexpr int COLS = 64 * V;
     constexpr bool PACKED = LbPacked<AK>::value;
-    static_assert(COLS == 256 || !PACKED, "one column of the tile per thread in the packed look-back");
-    constexpr int CH = int(kTileLbRows);
-    constexpr int RW = CH / 4;                  // rows per wave in a sub-tile
-    constexpr uint32_t SUB = 4u * RW;           // rows of a sub-tile
-    constexpr int NS = int(kTileLbRows / SUB);  // sub-tiles of a chunk, all held in registers
-    static_assert(NS == 1 && int(SUB) == CH, "a chunk is one sub-tile");
-    constexpr int HC = COLS / 2;                // TRANS: columns of one half of the tile in LDS
+    static_assert(COLS <= 256, "a thread per column of the tile in the look-back");
+    constexpr int CH = int(kTileLbRows);  // rows of a chunk with one row group a wave
+    constexpr int RW = CH / 4;            // rows a lane holds
+    constexpr int HC = COLS / 2;          // TRANS: columns of one half of the tile in LDS
     constexpr int PITCH = CH + 1;
     static_assert(!TRANS || NATIVE, "the transposed scan stores the input's type");
     union Shared {
-        Store wtot[NS][4][COLS];
+        Store wtot[4 * COLS];
         T tile[TRANS ? HC : 1][TRANS ? PITCH : 1];
     };
     __shared__ Shared sm;
@@ -225,6 +227,12 @@ __global__ __launch_bounds__(256) void scan_tiles_1p_kernel(const TileScan p) {
     __shared__ uint32_t s_ticket, s_depth, s_timed_out;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
+    const uint32_t L = TRANS ? 64u : p.lanes;       // lanes per row: a power of two, 4 .. 64
+    const uint32_t G = 64u / L;                     // row groups of a wave
+    const uint32_t cols = L * uint32_t(V);          // columns of the tile
+    const uint32_t lc = (uint32_t(lane) & (L - 1u)) * uint32_t(V);  // the lane's first column in it
+    const uint32_t sub = uint32_t(wave) * G + uint32_t(lane) / L;   // its row group, in row order
+    const uint32_t chunk_rows = uint32_t(CH) * G;
     const uint32_t cls = blockIdx.x % p.classes;
     if (threadIdx.x == 0) s_ticket = atomicAdd(p.ctrl + cls * kTileCtrlStride, 1u);
     __syncthreads();
@@ -236,10 +244,10 @@ __global__ __launch_bounds__(256) void scan_tiles_1p_kernel(const TileScan p) {
     const uint32_t chain = cls + p.classes * (i - chunk * per);
     const uint32_t tile = chain % p.ntiles;
     const uint32_t o = chain / p.ntiles;
-    const uint32_t col = tile * uint32_t(COLS) + uint32_t(lane * V);
+    const uint32_t col = tile * cols + lc;
     const int nv = col < p.inner ? min(V, int(p.inner - col)) : 0;
-    const uint32_t r0 = chunk * kTileLbRows;
-    const uint32_t r1 = min(p.len, r0 + kTileLbRows);
+    const uint32_t r0 = chunk * chunk_rows;
+    const uint32_t r1 = min(p.len, r0 + chunk_rows);
     const T* base = reinterpret_cast<const T*>(p.in) + int64_t(o) * p.in_s_outer + col;
     const int odt = NATIVE ? int(ScanInDtype<T>::value) : p.out_dtype;
     const int rdt = NATIVE ? int(ScanInDtype<T>::value) : p.rdt;
@@ -248,62 +256,54 @@ __global__ __launch_bounds__(256) void scan_tiles_1p_kernel(const TileScan p) {
     const bool nt_in = p.nt_in != 0, nt_out = p.nt_out != 0;
     A id;
     id.init(p.identity);
-    // the whole chunk: sub-tile s, wave w holds rows r0 + s*SUB + w*RW + [0, RW)
+    // the whole chunk: row group `sub` holds rows r0 + sub*RW + [0, RW)
     // (rows past the chunk clamped to its last row; their values are never used)
-    const bool whole = (tile + 1u) * uint32_t(COLS) <= p.inner;  // uniform in the block
-    T x[NS][RW][V];
+    const bool whole = (tile + 1u) * cols <= p.inner;  // uniform in the block
+    const uint32_t rw0 = r0 + sub * uint32_t(RW);
+    T x[RW][V];
+    if (whole && nt_in) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        const uint32_t rw0 = r0 + uint32_t(s) * SUB + uint32_t(wave * RW);
-        if (whole && nt_in) {
+        for (int i = 0; i < RW; ++i)
+            load_row<V, true>(base + int64_t(min(rw0 + uint32_t(i), r1 - 1)) * p.in_s_len, x[i]);
+    } else if (whole) {
 #pragma unroll
-            for (int i = 0; i < RW; ++i)
-                load_row<V, true>(base + int64_t(min(rw0 + uint32_t(i), r1 - 1)) * p.in_s_len, x[s][i]);
-        } else if (whole) {
+        for (int i = 0; i < RW; ++i)
+            load_row<V, false>(base + int64_t(min(rw0 + uint32_t(i), r1 - 1)) * p.in_s_len, x[i]);
+    } else {
+        load_rows_edge<RW, V>(base, p.in_s_len, rw0, 1u, r1, nv, x);
+    }
+    // every row group's total of every column
 #pragma unroll
-            for (int i = 0; i < RW; ++i)
-                load_row<V, false>(base + int64_t(min(rw0 + uint32_t(i), r1 - 1)) * p.in_s_len, x[s][i]);
-        } else {
+    for (int v = 0; v < V; ++v) {
+        A t = id;
 #pragma unroll
-            for (int i = 0; i < RW; ++i) {
-                const uint32_t row = rw0 + uint32_t(i);
-                load_row_partial<V>(base + int64_t(min(row, r1 - 1)) * p.in_s_len, row < r1, nv, x[s][i]);
+        for (int i = 0; i < RW; ++i)
+            if (rw0 + uint32_t(i) < r1) t.add(reg_put<T>(x[i][v]));
+        sm.wtot[sub * cols + lc + uint32_t(v)] = t.store();
+    }
+    __syncthreads();
+    // thread c: column c of the tile.  The groups' totals become exclusive
+    // prefixes inside the chunk, in place; then the look-back.
+    const uint32_t c = threadIdx.x;
+    const bool has_col = c < cols;
+    A agg = id, excl = id;
+    if (has_col) {
+        for (uint32_t s = 0; s < 4u * G; s += 4u) {
+            A t[4];
+#pragma unroll
+            for (uint32_t w = 0; w < 4u; ++w) t[w].load(sm.wtot[(s + w) * cols + c]);
+#pragma unroll
+            for (uint32_t w = 0; w < 4u; ++w) {
+                sm.wtot[(s + w) * cols + c] = agg.store();
+                agg.merge(t[w]);
             }
         }
     }
-    // every (sub-tile, wave) total of every column
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        const uint32_t rw0 = r0 + uint32_t(s) * SUB + uint32_t(wave * RW);
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-            A t = id;
-#pragma unroll
-            for (int i = 0; i < RW; ++i)
-                if (rw0 + uint32_t(i) < r1) t.add(reg_put<T>(x[s][i][v]));
-            sm.wtot[s][wave][lane * V + v] = t.store();
-        }
-    }
-    __syncthreads();
-    if constexpr (!PACKED) {  // thread c < COLS: column c; value, wait, flag per (chunk, tile)
-        const int c = int(threadIdx.x);
-        const bool has_col = c < COLS;
-        A agg = id;
-        if (has_col) {
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    A t;
-                    t.load(sm.wtot[s][w][c]);
-                    agg.merge(t);
-                }
-        }
-        const int64_t vbase = int64_t(o) * p.nchunks * p.ncols + tile * uint32_t(COLS) + (has_col ? c : 0);
+    if constexpr (!PACKED) {  // value, wait, flag per (chunk, tile)
+        const int64_t vbase = int64_t(o) * p.nchunks * p.ncols + tile * cols + (has_col ? c : 0u);
         uint32_t* ftile = p.flags + int64_t(o) * p.nchunks * p.ntiles + tile;
         uint32_t* fmine = ftile + int64_t(chunk) * p.ntiles;
         const int64_t vmine = vbase + int64_t(chunk) * p.ncols;
-        A excl = id;
         if (chunk == 0) {  // uniform in the block
             tile_publish_flagged<AK, OP>(p.pre + vmine, has_col, agg, fmine, kLbPrefix);
         } else {
@@ -325,129 +325,103 @@ __global__ __launch_bounds__(256) void scan_tiles_1p_kernel(const TileScan p) {
             incl.merge(agg);
             tile_publish_flagged<AK, OP>(p.pre + vmine, has_col, incl, fmine, kLbPrefix);
         }
-        if (has_col) s_excl[c] = excl.store();
-    } else {  // thread c: column c of the tile, the chunk's total, look-back, publications
-        const int c = int(threadIdx.x);
-        A agg = id;
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                A t;
-                t.load(sm.wtot[s][w][c]);
-                agg.merge(t);
-            }
-        uint64_t* wtile = p.words + int64_t(o) * p.nchunks * p.ncols + tile * uint32_t(COLS);
-        uint64_t* mine = wtile + int64_t(chunk) * p.ncols + c;
-        A excl = id;
+    } else {
+        uint64_t* wtile = p.words + int64_t(o) * p.nchunks * p.ncols + tile * cols;
+        uint64_t* mine = wtile + int64_t(chunk) * p.ncols + (has_col ? c : 0u);
         if (chunk == 0) {  // uniform in the block
-            lb_store(mine, lb_pack(agg, kLbPrefix));
+            if (has_col) lb_store(mine, lb_pack(agg, kLbPrefix));
         } else {
-            lb_store(mine, lb_pack(agg, kLbAggregate));
+            if (has_col) lb_store(mine, lb_pack(agg, kLbAggregate));
             if (wave == 0) {
                 const uint32_t d = tile_lead_depth(wtile, p.ncols, chunk);
                 if (lane == 0) s_depth = d;
             }
             __syncthreads();
-            excl = tile_follow<AK, OP>(wtile + c, p.ncols, chunk, s_depth, id, p.ctrl + kTileTimeouts);
-            A incl = excl;
-            incl.merge(agg);
-            lb_store(mine, lb_pack(incl, kLbPrefix));
+            if (has_col) {
+                excl = tile_follow<AK, OP>(wtile + c, p.ncols, chunk, s_depth, id, p.ctrl + kTileTimeouts);
+                A incl = excl;
+                incl.merge(agg);
+                lb_store(mine, lb_pack(incl, kLbPrefix));
+            }
         }
-        s_excl[c] = excl.store();
     }
+    if (has_col) s_excl[c] = excl.store();
     __syncthreads();
-    // each lane's start for every sub-tile: the chunk's carry, then the
-    // (sub-tile, wave) totals before it in row order
-    A pre[NS][V];
+    // each lane's start: the chunk's carry, then the row groups before its own
+    A run[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
-        A carry;
-        carry.load(s_excl[lane * V + v]);
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                A t;
-                t.load(sm.wtot[s][w][lane * V + v]);
-                if (w == wave) pre[s][v] = carry;
-                carry.merge(t);
-            }
+        A t;
+        run[v].load(s_excl[lc + uint32_t(v)]);
+        t.load(sm.wtot[sub * cols + lc + uint32_t(v)]);
+        run[v].merge(t);
     }
-    __syncthreads();  // wtot is read; the transposed form reuses the space
+    if constexpr (!TRANS) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        const uint32_t sub = r0 + uint32_t(s) * SUB;
-        const uint32_t rw0 = sub + uint32_t(wave * RW);
-        A run[V];
+        for (int i = 0; i < RW; ++i) {
+            const uint32_t row = rw0 + uint32_t(i);
+            if (row >= r1) continue;
+            Reg y[V];
 #pragma unroll
-        for (int v = 0; v < V; ++v) run[v] = pre[s][v];
-        if constexpr (!TRANS) {
+            for (int v = 0; v < V; ++v) {
+                run[v].add(reg_put<T>(x[i][v]));
+                const Reg val = run[v].value(rdt);
+                if constexpr (NATIVE) y[v] = val;
+                else y[v] = cvt(val, rdt, odt);
+            }
+            char* ptr = obase + (int64_t(row) * p.out_s_len + int64_t(col) * p.out_s_inner) * oesz;
+            if (nv == V) {
+                store_vec_rt(nt_out, ptr, oesz, odt, y);
+            } else {
 #pragma unroll
-            for (int i = 0; i < RW; ++i) {
-                const uint32_t row = rw0 + uint32_t(i);
-                if (row >= r1) continue;  // uniform in the wave
-                Reg y[V];
+                for (int v = 0; v < V; ++v)
+                    if (v < nv) store_raw(ptr + int64_t(v) * p.out_s_inner * oesz, oesz, y[v]);
+            }
+        }
+    } else {
+        __syncthreads();  // wtot is read; its space is reused
+        // the results in place of the values, then the chunk as [column][row] in
+        // LDS in two halves of 128 columns (lanes 0-31, then 32-63), each stored
+        // along the output's rows: a column's 64 rows are one 256-byte segment
 #pragma unroll
-                for (int v = 0; v < V; ++v) {
-                    run[v].add(reg_put<T>(x[s][i][v]));
-                    const Reg val = run[v].value(rdt);
-                    if constexpr (NATIVE) y[v] = val;
-                    else y[v] = cvt(val, rdt, odt);
-                }
-                char* ptr = obase + (int64_t(row) * p.out_s_len + int64_t(col) * p.out_s_inner) * oesz;
-                if (nv == V) {
-                    store_vec_rt(nt_out, ptr, oesz, odt, y);
+        for (int i = 0; i < RW; ++i) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                if (rw0 + uint32_t(i) < r1) run[v].add(reg_put<T>(x[i][v]));
+                x[i][v] = reg_get<T>(run[v].value(rdt));
+            }
+        }
+        constexpr int TPC = CH / V;     // threads per column: 16 bytes each
+        constexpr int CPP = 256 / TPC;  // columns per pass
+        const int cc = threadIdx.x / TPC;
+        const int rr = (threadIdx.x - cc * TPC) * V;
+        const uint32_t row = r0 + uint32_t(rr);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if ((lane >> 5) == h) {
+#pragma unroll
+                for (int i = 0; i < RW; ++i)
+#pragma unroll
+                    for (int v = 0; v < V; ++v) sm.tile[(lane & 31) * V + v][wave * RW + i] = x[i][v];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int c = cc; c < HC; c += CPP) {
+                const uint32_t gcol = tile * uint32_t(COLS) + uint32_t(h * HC + c);
+                if (gcol >= p.inner || row >= r1) continue;
+                char* ptr = obase + (int64_t(row) * p.out_s_len + int64_t(gcol) * p.out_s_inner) * oesz;
+                Reg q[V];
+#pragma unroll
+                for (int v = 0; v < V; ++v) q[v] = reg_put<T>(sm.tile[c][rr + v]);
+                if (row + uint32_t(V) <= r1) {
+                    store_vec_rt(nt_out, ptr, oesz, odt, q);
                 } else {
 #pragma unroll
                     for (int v = 0; v < V; ++v)
-                        if (v < nv) store_raw(ptr + int64_t(v) * p.out_s_inner * oesz, oesz, y[v]);
+                        if (row + uint32_t(v) < r1) store_raw(ptr + int64_t(v) * oesz, oesz, q[v]);
                 }
             }
-        } else {
-            // the results in place of the values, then the chunk as [column][row] in
-            // LDS in two halves of 128 columns (lanes 0-31, then 32-63), each stored
-            // along the output's rows: a column's 64 rows are one 256-byte segment
-#pragma unroll
-            for (int i = 0; i < RW; ++i) {
-#pragma unroll
-                for (int v = 0; v < V; ++v) {
-                    if (rw0 + uint32_t(i) < r1) run[v].add(reg_put<T>(x[s][i][v]));
-                    x[s][i][v] = reg_get<T>(run[v].value(rdt));
-                }
-            }
-            constexpr int TPC = CH / V;     // threads per column: 16 bytes each
-            constexpr int CPP = 256 / TPC;  // columns per pass
-            const int cc = threadIdx.x / TPC;
-            const int rr = (threadIdx.x - cc * TPC) * V;
-            const uint32_t row = sub + uint32_t(rr);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                if ((lane >> 5) == h) {
-#pragma unroll
-                    for (int i = 0; i < RW; ++i)
-#pragma unroll
-                        for (int v = 0; v < V; ++v) sm.tile[(lane & 31) * V + v][wave * RW + i] = x[s][i][v];
-                }
-                __syncthreads();
-#pragma unroll
-                for (int c = cc; c < HC; c += CPP) {
-                    const uint32_t gcol = tile * uint32_t(COLS) + uint32_t(h * HC + c);
-                    if (gcol >= p.inner || row >= r1) continue;
-                    char* ptr = obase + (int64_t(row) * p.out_s_len + int64_t(gcol) * p.out_s_inner) * oesz;
-                    Reg q[V];
-#pragma unroll
-                    for (int v = 0; v < V; ++v) q[v] = reg_put<T>(sm.tile[c][rr + v]);
-                    if (row + uint32_t(V) <= r1) {
-                        store_vec_rt(nt_out, ptr, oesz, odt, q);
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < V; ++v)
-                            if (row + uint32_t(v) < r1) store_raw(ptr + int64_t(v) * oesz, oesz, q[v]);
-                    }
-                }
-                __syncthreads();  // the tile space is written again for the second half
-            }
+            __syncthreads();  // the tile space is written again for the second half
         }
     }
 }
