@@ -44,6 +44,10 @@ HIP_FLAGS = [
     "-I", INCLUDE,
 ]
 
+# Per source: the interpreter's op dispatch branches on wave-uniform values
+# only; without this the compiler rebuilds it as cascades of flag tests.
+FILE_FLAGS = {"ew_interp.hip": ["-mllvm", "-structurizecfg-skip-uniform-regions"]}
+
 
 HOST_FLAGS = [
     "-O2",
@@ -102,7 +106,7 @@ def build(force: bool = False, jobs: int | None = None) -> str:
         objs.append(o)
         if force or not os.path.exists(o) or max(os.path.getmtime(s), hdr_time) > os.path.getmtime(o):
             if s.endswith(".hip"):
-                todo.append([HIPCC] + HIP_FLAGS + ["-x", "hip", "-c", s, "-o", o])
+                todo.append([HIPCC] + HIP_FLAGS + FILE_FLAGS.get(os.path.basename(s), []) + ["-x", "hip", "-c", s, "-o", o])
             else:  # host-only translation units
                 todo.append(["g++"] + HOST_FLAGS + ["-c", s, "-o", o])
     if todo:

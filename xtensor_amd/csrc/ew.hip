@@ -20,72 +20,6 @@
 #include "jit.hpp"
 #include "planner.hpp"
 
-namespace xg {
-
-template <int V, bool I64>
-__device__ __forceinline__ void store_out(const EwPlan& plan, int mode, int dt, const uint32_t* idx, uint32_t j0,
-                                          int nvalid, const Reg (&val)[V]) {
-    const int esz = dtype_size(dt);
-    auto off = unit_offset<I64>(plan.out_stride, idx, plan.rank, j0);
-    char* p = plan.out_ptr + int64_t(off) * esz;
-    if (mode == LM_CONTIG && nvalid == V) {
-        store_vec<V>(p, esz, dt, val);
-    } else {
-        const int64_t os = plan.out_stride[plan.rank - 1];
-#pragma unroll
-        for (int v = 0; v < V; ++v)
-            if (v < nvalid) store_raw(p + int64_t(v) * os * esz, esz, to_storage(val[v], dt));
-    }
-}
-
-// The generic interpreter for elementwise plans of vector width 1: one
-// element per work item and the program's register file in LDS, indexed
-// [register][thread] (a register array indexed by run-time operands would
-// live in scratch memory).  Each micro-op is one out-of-line call.
-template <bool I64>
-__global__ __launch_bounds__(256) void ew_lds_kernel(const EwPlan plan_arg) {
-    const EwPlan& plan = kernel_plan<DynSpec>(plan_arg);
-    __shared__ Reg regs[kMaxRegs][256];
-    const int tid = int(threadIdx.x);
-    const uint32_t nunits = uint32_t(plan.units);
-    const uint32_t step = gridDim.x * 256u;
-    for (uint32_t u = blockIdx.x * 256u + uint32_t(tid); u < nunits; u += step) {
-        const uint32_t row = fastdiv(u, plan.div_chunks);
-        const uint32_t j0 = u - row * plan.nchunks;
-        uint32_t idx[kMaxRank];
-        uint32_t r = row;
-#pragma unroll
-        for (int k = kMaxRank - 2; k >= 0; --k) {
-            if (k <= plan.rank - 2) {
-                const uint32_t q = fastdiv(r, plan.div[k]);
-                idx[k] = r - q * uint32_t(plan.shape[k]);
-                r = q;
-            } else {
-                idx[k] = 0;
-            }
-        }
-        for (int pc = 0; pc < plan.prog.nops; ++pc) {
-            const MicroOp m = plan.prog.ops[pc];
-            Reg v[1];
-            if (m.op == MO_LOAD) {
-                const LeafView& lv = plan.leaves[m.aux];
-                load_leaf<1, I64>(lv, lv.mode, lv.dtype, idx, plan.rank, j0, 1, v);
-            } else if (m.op == MO_GATHER) {
-                const LeafView& lv = plan.leaves[m.aux];
-                const Reg off[1] = {regs[m.a][tid]};
-                gather_vals<1>(lv.ptr, lv.dtype, lv.stride[0], lv.stride[1], 1, off, v);
-            } else {
-                v[0] = exec_scalar_dyn(m, regs[m.a][tid], regs[m.b][tid], regs[m.c][tid], plan.prog.consts);
-            }
-            regs[m.dst][tid] = v[0];
-        }
-        const Reg res[1] = {regs[plan.prog.result_reg][tid]};
-        store_out<1, I64>(plan, lm_base(plan.out_mode), plan.out_dtype, idx, j0, 1, res);
-    }
-}
-
-}  // namespace xg
-
 // compiled specialisations (generated from specs_list.cpp at build time)
 #include "specs.inc"
 
@@ -248,11 +182,8 @@ hipError_t launch_ew(const EwPlan& p, int V, int cus, hipStream_t stream, const 
         if (used) *used = k->name.c_str();
         return jit_launch(k, grid.x, 256, &p, sizeof(EwPlan), stream);
     }
-    if (V != 1) return hipErrorInvalidValue;  // the generic interpreter takes one element per lane
     if (used) *used = "dynamic";
-    if (p.index64) hipLaunchKernelGGL((ew_lds_kernel<true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((ew_lds_kernel<false>), grid, block, 0, stream, p);
-    return hipGetLastError();
+    return launch_ew_interp(p, V, grid, stream);
 }
 
 }  // namespace xg

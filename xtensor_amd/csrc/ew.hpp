@@ -11,6 +11,8 @@ namespace xg {
 // Launch out = program(leaves) for a plan built with vector width V.
 // `used` (optional) receives the name of the kernel that ran.
 hipError_t launch_ew(const EwPlan& p, int V, int cus, hipStream_t stream, const char** used);
+// The same by the generic interpreter (V = ew_interp_width(p)).
+hipError_t launch_ew_interp(const EwPlan& p, int V, dim3 grid, hipStream_t stream);
 #endif
 
 // Name of the compiled specialisation that matches the plan, or nullptr.
@@ -24,6 +26,9 @@ int ew_set_thread_force_dynamic(int on);
 // True when a plan without an ahead-of-time program runs a run-time compiled
 // one (compiling it on first use).
 bool ew_jit_ok(const EwPlan& p, int V);
+// Vector width the generic interpreter takes the plan's program at (the plan
+// is to be made with it).
+int ew_interp_width(const EwPlan& p);
 // Force one (1) or four (4) work units per thread in compiled kernels, or
 // choose by size (0) (measurement aid).
 void ew_set_units_per_thread(int upt);

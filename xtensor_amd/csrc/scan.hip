@@ -28,7 +28,8 @@ hipError_t launch_scan(const ScanPlan& p, int V, void* ws, hipStream_t stream, c
     if (p.rows == 0) return hipSuccess;
     if (V != 4) return hipErrorInvalidValue;
     ScanKernels k{};
-    if (!scan_kernels_float(p.acc, p.op, &k) && !scan_kernels_int(p.acc, p.op, &k)) return hipErrorInvalidValue;
+    if (!scan_kernels_float(p.acc, p.op, &k) && !scan_kernels_int(p.acc, p.op, &k) && !scan_kernels_long(p.acc, p.op, &k))
+        return hipErrorInvalidValue;
     dim3 block(256);
     if (p.tiled == ST_SHORT) {
         TFn f = k.shorts[p.tile_native ? 1 : 0];

@@ -1,4 +1,4 @@
-// scan_int.hip — scan kernel instantiations for one accumulator family.
+// scan_int.hip — scan kernel instantiations for the 32-bit integer accumulators.
 #include "scan_kernels.hpp"
 
 namespace xg {
@@ -9,10 +9,6 @@ bool scan_kernels_int(int ak, int op, ScanKernels* k) {
     XG_S(AK_I32, RO_MUL)
     XG_S(AK_U32, RO_ADD)
     XG_S(AK_U32, RO_MUL)
-    XG_S(AK_I64, RO_ADD)
-    XG_S(AK_I64, RO_MUL)
-    XG_S(AK_U64, RO_ADD)
-    XG_S(AK_U64, RO_MUL)
 #undef XG_S
     return false;
 }

@@ -395,5 +395,6 @@ template <int AK, int OP> ScanKernels scan_kernels() {
 
 bool scan_kernels_float(int ak, int op, ScanKernels* k);
 bool scan_kernels_int(int ak, int op, ScanKernels* k);
+bool scan_kernels_long(int ak, int op, ScanKernels* k);
 
 }  // namespace xg
