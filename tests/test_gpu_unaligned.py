@@ -74,3 +74,34 @@ def test_reduce_inner_view(dtype, tol, axis, rows, pitch, c0, cols):
     assert np.all(np.abs(got.astype(np.float64) - ref) <= tol * mag)
     m = xt.amax(v.dev, [axis])
     assert same_bits(xt.eval(m).to_numpy(), o.reduce(m))
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32", "float64", "int32"])
+@pytest.mark.parametrize("shape,axes", [((3, 5, 7, 7), [0, 2, 3]), ((9, 2, 1, 3), [0, 2, 3]), ((33, 1, 5, 13), [0, 2, 3]),
+                                        ((130, 300, 2, 9), [0, 2, 3]), ((1, 700, 3, 3), [0, 2, 3]), ((5, 1001), [0]),
+                                        ((2000, 131), [0]), ((1100, 520), [0]), ((70, 3), [0, 1])])
+def test_channel_and_ragged_reductions(dtype, shape, axes):
+    """Rows of [outputs | reduced | fast], columns whose last chunk is shifted,
+    one output, rows shorter than a vector: sums within one rounding relative
+    to the sum of magnitudes (as above), maxima and infinities exact."""
+    rng = np.random.default_rng(sum(shape))
+    h = rng.integers(-1000, 1000, shape).astype("int32") if dtype == "int32" else \
+        rng.normal(size=shape).astype("float32" if dtype == "bfloat16" else dtype)
+    d = Dual.of(h, dtype if dtype == "bfloat16" else None)
+    o = oracle_for(d)
+    r = xt.sum(d.dev, axes)
+    got = xt.eval(r).to_numpy()
+    if dtype == "int32":
+        assert same_bits(got, o.reduce(r))
+    else:
+        mag = o.reduce(xt.sum(xt.abs(d.dev), axes), high_precision=True)
+        tol = 1e-15 if dtype == "float64" else 1e-7
+        assert np.all(np.abs(got.astype(np.float64) - o.reduce(r, high_precision=True)) <= tol * mag)
+    for m in (xt.amax(d.dev, axes), xt.amin(d.dev, axes)):
+        assert same_bits(xt.eval(m).to_numpy(), o.reduce(m))
+    if dtype in ("float32", "float64"):
+        h2 = np.full(shape, -np.inf, dtype)  # folds to lowest(), but where the infinity is
+        h2.reshape(-1)[-1] = np.inf
+        d2 = Dual.of(h2)
+        m = xt.amax(d2.dev, axes)
+        assert same_bits(xt.eval(m).to_numpy(), oracle_for(d2).reduce(m))

@@ -353,6 +353,7 @@ const JitKernel* jit_reduce(const RedPlan& p, int V, int kind) {
     switch (kind) {
     case JR_ROWS_FAST1: expr = "&xg::reduce_rows_fast_kernel<" + head + ao + ", 1>"; break;
     case JR_ROWS_FAST2: expr = "&xg::reduce_rows_fast_kernel<" + head + ao + ", 2>"; break;
+    case JR_ROWS_FAST3: expr = "&xg::reduce_rows_fast_kernel<" + head + ao + ", 3>"; break;
     case JR_COLS_FAST: expr = "&xg::reduce_cols_fast_kernel<" + head + ao + ">"; break;
     case JR_ROWS: expr = "&xg::reduce_rows_kernel<" + head + "false, " + ao + ", 4>"; break;
     case JR_COLS: expr = "&xg::reduce_cols_kernel<" + head + "false, " + ao + ", 4>"; break;

@@ -20,7 +20,7 @@
 namespace xg {
 
 // which kernel template of a reduction plan
-enum JitRedKind : int { JR_ROWS_FAST1 = 0, JR_ROWS_FAST2, JR_COLS_FAST, JR_ROWS, JR_COLS };
+enum JitRedKind : int { JR_ROWS_FAST1 = 0, JR_ROWS_FAST2, JR_ROWS_FAST3, JR_COLS_FAST, JR_ROWS, JR_COLS };
 
 struct JitKernel {
     hipFunction_t fn = nullptr;

@@ -117,7 +117,8 @@ uint64_t plan_elements(const RedPlan& p) {
 
 // the kernel template a plan runs: a fast one for compact plans
 int jit_kind(const RedPlan& p) {
-    if (p.compact) return p.layout == RL_ROWS ? (p.rank == 1 ? JR_ROWS_FAST1 : JR_ROWS_FAST2) : JR_COLS_FAST;
+    if (p.compact)
+        return p.layout != RL_ROWS ? JR_COLS_FAST : p.f_rank == 1 ? JR_ROWS_FAST1 : p.f_rank == 2 ? JR_ROWS_FAST2 : JR_ROWS_FAST3;
     return p.layout == RL_ROWS ? JR_ROWS : JR_COLS;
 }
 
@@ -151,8 +152,8 @@ hipError_t launch_reduce(RedPlan& p, int V, hipStream_t stream, const char** use
         hipLaunchKernelGGL(f, dim3(grid), dim3(block), 0, stream, q);
         return hipGetLastError();
     };
-    const bool fast = p.compact &&
-                      (jk || (sp && (p.layout == RL_ROWS ? (p.rank == 1 ? ks.rows_fast1 : ks.rows_fast2) : ks.cols_fast)));
+    KFn rows_fast = p.f_rank == 1 ? ks.rows_fast1 : p.f_rank == 2 ? ks.rows_fast2 : ks.rows_fast3;
+    const bool fast = p.compact && (jk || (sp && (p.layout == RL_ROWS ? rows_fast : ks.cols_fast)));
     if (fast) {
         // compiled fast kernels with their own split of the work
         RedPlan q = p;
@@ -166,7 +167,7 @@ hipError_t launch_reduce(RedPlan& p, int V, hipStream_t stream, const char** use
             const uint64_t per_block = 4 * (64 / uint64_t(q.group));
             const uint64_t blocks = (items + per_block - 1) / per_block;
             if (blocks >= (uint64_t(1) << 31)) return hipErrorInvalidValue;
-            err = go(q.rank == 1 ? ks.rows_fast1 : ks.rows_fast2, uint32_t(blocks), 256, q);
+            err = go(rows_fast, uint32_t(blocks), 256, q);
         } else {
             const uint64_t tw = uint64_t(q.group);  // tile width in lanes
             if (tw != 64 && tw != 128 && tw != 256) return hipErrorInvalidValue;
@@ -184,7 +185,7 @@ hipError_t launch_reduce(RedPlan& p, int V, hipStream_t stream, const char** use
             // once and the merges then run on a few workgroups, latency-bound
             // (float32 [8192, 4096] column sum 31 -> 45 us, bf16 27 -> 81 us).
             q.counters = nullptr;
-            err = go(ks.cols_fast, uint32_t(blocks), 512, q);
+            err = go(ks.cols_fast, uint32_t(blocks), kColsBlock, q);
         }
         if (err != hipSuccess || q.splits == 1) return err;
         return launch_combine(q, stream);

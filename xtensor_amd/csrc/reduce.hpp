@@ -39,6 +39,9 @@ enum Finalize : int32_t { FZ_NONE = 0, FZ_MEAN = 1, FZ_SQRT = 2, FZ_MEAN_SQRT = 
 constexpr int kRedMinNum = 100;
 constexpr int kRedMaxNum = 101;
 
+// threads of a block of the column fast kernel
+constexpr int kColsBlock = 1024;
+
 struct RedPlan {
     int32_t layout;
     int32_t rank;       // normalised dims (see below)
@@ -84,10 +87,12 @@ struct RedPlan {
     int32_t combine_group;
     LeafView leaves[kMaxLeaves];
     Program prog;       // element value mapped and converted to the accumulation type
-    // Compact form for the compiled fast kernels: normalised rank <= 2 and
-    // 32-bit offsets (rows: [outputs | fast] or [fast]; cols: [rows | fast]).
-    // cst[l][k] = stride of leaf l along dim k.  f_* = their work split.
+    // Compact form for the compiled fast kernels and 32-bit offsets: rows of
+    // f_rank 1 [fast], 2 [outputs | fast] or 3 [outputs | reduced | fast] (one
+    // output: stride 0 in front), cols [rows | fast].  cst[l][k] = stride of
+    // leaf l along dim k of that form.  f_* = their work split.
     int32_t compact;
+    int32_t f_rank;
     int32_t f_group;      // rows: lanes per output (1..64, power of two); cols: tile width in lanes (64, 128, 256)
     int32_t f_splits;     // partial results per output
     uint32_t f_per_split; // rows: chunks per split; cols: rows per split

@@ -365,7 +365,7 @@ __global__ __launch_bounds__(256) void reduce_combine_wide_kernel(const RedPlan 
 }
 
 // ---------------------------------------------------------------- compiled fast kernels
-// For compact plans (normalised rank <= 2, 32-bit offsets) and a compiled
+// For compact plans (rows of normalised rank <= 3, columns of rank 2, 32-bit offsets) and a compiled
 // program: leaf offsets are one multiply-add per dimension, U chunks (rows)
 // are in flight per lane, and the rows kernel combines inside a wave only
 // (no LDS, no barrier).  p.group / p.splits / p.per_split hold the fast
@@ -392,7 +392,14 @@ template <int NR, int V, bool COLS> constexpr int fast_unroll() {
     return NR * V <= 8 ? 4 : (NR * V <= 16 ? 2 : 1);
 }
 
-// rows: dims [outputs | fast] (RANK 2) or [fast] (RANK 1, one output);
+// Ragged rows (lf no multiple of V): the last chunk of a row is read as the
+// row's last V elements and the leading ones, which the chunk before it holds,
+// are dropped with a select, so that no load sits behind a lane-dependent
+// branch.  bf16 [5003, 3001], V = 8, a launch and its merge: row means 12.7 ->
+// 11.1 us, column means 50.7 -> 20.0 us (with the block and split rules below).
+
+// rows: dims [outputs | fast] (RANK 2), [fast] (RANK 1, one output) or
+// [outputs | reduced | fast] (RANK 3: a channel's images);
 // G lanes per (output, split), 64 / G of them per wave
 template <int V, int NR, class S, int AK, int OP, int RANK>
 __global__ __launch_bounds__(256) void reduce_rows_fast_kernel(const RedPlan p) {
@@ -410,49 +417,77 @@ __global__ __launch_bounds__(256) void reduce_rows_fast_kernel(const RedPlan p) 
     const uint32_t o = live ? fastdiv(wi, p.div_splits) : 0u;
     const uint32_t sp = wi - o * uint32_t(p.splits);
     const uint32_t c0 = sp * p.per_split;
-    const uint32_t c1 = live ? min(p.nchunks_f, c0 + p.per_split) : 0u;
-    const uint32_t idx[4] = {RANK == 2 ? o : 0u, 0u, 0u, 0u};
-    // FULL: every chunk of the lane's range is whole, so chunks past the
-    // range's end are clamped to its last chunk and their values dropped,
-    // and no load sits behind a divergent branch (U loads stay in flight)
-    auto sweep = [&](auto full_c, auto ntm_c) {
-        constexpr bool FULL = decltype(full_c)::value;
+    const uint32_t c1 = live ? min(p.red_count, c0 + p.per_split) : 0u;
+    // the row and the first element of chunk c
+    auto place = [&](uint32_t c, uint32_t (&idx)[4], uint32_t& j0) {
+        uint32_t ro = 0;
+        if constexpr (RANK == 3) ro = fastdiv(c, p.div_nchunks_f);
+        j0 = (c - ro * p.nchunks_f) * V;
+        idx[0] = RANK >= 2 ? o : 0u;
+        idx[1] = ro;
+        idx[2] = idx[3] = 0u;
+    };
+    // rows of at least V elements: chunks past the lane's range are clamped to
+    // its last one and their values dropped (U loads stay in flight)
+    auto sweep = [&](auto ragged_c, auto ntm_c) {
+        constexpr bool RAGGED = decltype(ragged_c)::value;
         constexpr int NTM = decltype(ntm_c)::value;
         for (uint32_t c = c0 + gl; c < c1; c += uint32_t(G) * U) {
             Reg R[U][NR][V];
-            int nv[U];
+            bool ok[U];
+            uint32_t drop[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const uint32_t cc = c + uint32_t(u * G);
-                if constexpr (FULL) {
-                    nv[u] = cc < c1 ? V : 0;
-                    run_spec<S, 0, V, NR, RANK, true, NTM>(p, idx, min(cc, c1 - 1) * V, V, R[u]);
-                } else {
-                    nv[u] = cc < c1 ? min(V, int(p.lf - cc * V)) : 0;
-                    if (nv[u] > 0) run_spec<S, 0, V, NR, RANK>(p, idx, cc * V, nv[u], R[u]);
+                ok[u] = cc < c1;
+                uint32_t idx[4], j0;
+                place(min(cc, c1 - 1), idx, j0);
+                drop[u] = 0;
+                if constexpr (RAGGED) {
+                    const uint32_t j = min(j0, p.lf - uint32_t(V));
+                    drop[u] = j0 - j;
+                    j0 = j;
                 }
+                run_spec<S, 0, V, NR, RANK, true, NTM>(p, idx, j0, V, R[u]);
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if constexpr (FULL) {  // a select, not a branch (see the cols kernel)
+            for (int u = 0; u < U; ++u) {  // selects, not branches (see the cols kernel)
+                if constexpr (RAGGED) {
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        A t = acc;
+                        t.add(R[u][S::result_reg][v]);
+                        acc = ok[u] && uint32_t(v) >= drop[u] ? t : acc;
+                    }
+                } else {
                     A t = acc;
 #pragma unroll
                     for (int v = 0; v < V; ++v) t.add(R[u][S::result_reg][v]);
-                    acc = nv[u] > 0 ? t : acc;
-                } else {
-#pragma unroll
-                    for (int v = 0; v < V; ++v)
-                        if (v < nv[u]) acc.add(R[u][S::result_reg][v]);
+                    acc = ok[u] ? t : acc;
                 }
             }
         }
     };
-    // whole chunks up to the lane's range end (or an empty range): uniform over the wave
-    const bool full = __all(c1 <= c0 || c1 * uint32_t(V) <= p.lf);
     const int ntm = spec_leaves_nt<S>(p);
-    if (full && ntm == 1) sweep(std::true_type{}, std::integral_constant<int, 1>{});
-    else if (full && ntm == 0) sweep(std::true_type{}, std::integral_constant<int, 0>{});
-    else sweep(std::false_type{}, std::integral_constant<int, 2>{});
+    if (p.lf >= uint32_t(V)) {  // uniform
+        const bool ragged = p.lf % uint32_t(V) != 0;
+        if (!ragged && ntm == 1) sweep(std::false_type{}, std::integral_constant<int, 1>{});
+        else if (!ragged && ntm == 0) sweep(std::false_type{}, std::integral_constant<int, 0>{});
+        else if (!ragged) sweep(std::false_type{}, std::integral_constant<int, 2>{});
+        else if (ntm == 1) sweep(std::true_type{}, std::integral_constant<int, 1>{});
+        else sweep(std::true_type{}, std::integral_constant<int, 2>{});
+    } else {
+        for (uint32_t c = c0 + gl; c < c1; c += uint32_t(G)) {
+            Reg R[NR][V];
+            uint32_t idx[4], j0;
+            place(c, idx, j0);
+            const int nv = int(p.lf - j0);
+            run_spec<S, 0, V, NR, RANK>(p, idx, j0, nv, R);
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+                if (v < nv) acc.add(R[S::result_reg][v]);
+        }
+    }
     acc = wave_group_combine(acc, G);
     if (live && gl == 0) {
         if (p.splits == 1) finish(p, acc, o);
@@ -460,17 +495,25 @@ __global__ __launch_bounds__(256) void reduce_rows_fast_kernel(const RedPlan p) 
     }
 }
 
-// cols: dims [rows | fast outputs]; a block of 512 threads = one tile of
+// cols: dims [rows | fast outputs]; a block of kColsBlock threads = one tile of
 // TW * V adjacent outputs (TW = p.group lanes: 64, 128 or 256) and one split
-// of the rows.  The block's 512 / TW row groups interleave rows, each lane
-// with U rows in flight, and combine in LDS in row-group order.
+// of the rows.  The block's kColsBlock / TW row groups interleave rows, each
+// lane with U rows in flight, and combine in LDS: the upper half of the block
+// into the lower, then in row-group order.  Bound by the loads in flight (a
+// CU needs ~50 KB of them to cover HBM's latency at its share of 5.5 TB/s):
+// 1024 threads hold twice what 512 do for the same number of partial results,
+// which two blocks of 512 would double (float32 column sums: [60000, 37] 27.1
+// -> 13.2 us, [500, 20001] 26.4 -> 16.7, [8192, 4096] 28.6 -> 29.4).  Lanes past
+// the last column, and the leading columns of the last lane's shifted chunk
+// (ragged rows), repeat columns of other lanes and are not written.
 template <int V, int NR, class S, int AK, int OP>
-__global__ __launch_bounds__(512) void reduce_cols_fast_kernel(const RedPlan p) {
+__global__ __launch_bounds__(kColsBlock) void reduce_cols_fast_kernel(const RedPlan p) {
     using A = Acc<AK, OP>;
     constexpr int U = fast_unroll<NR, V, true>();
-    __shared__ typename A::Lds lds[512][V];  // 8-byte pairs: a bf16 tile (V = 8) takes 32 KiB
+    constexpr uint32_t HB = kColsBlock / 2;
+    __shared__ typename A::Lds lds[HB][V];  // 8-byte pairs: a bf16 tile (V = 8) takes 32 KiB
     const uint32_t TW = uint32_t(p.group);
-    const uint32_t RG = 512u / TW;
+    const uint32_t RG = uint32_t(kColsBlock) / TW;
     const uint32_t tl = threadIdx.x & (TW - 1);
     const uint32_t rg = threadIdx.x / TW;
     // split fastest: the splits of one column strip run side by side (measured
@@ -480,18 +523,19 @@ __global__ __launch_bounds__(512) void reduce_cols_fast_kernel(const RedPlan p) 
     const uint32_t sp = blockIdx.x - tile * uint32_t(p.splits);
     const uint32_t cc = tile * TW + tl;
     const bool active = cc < p.nchunks_f;
-    const uint32_t j0 = cc * V;
+    const bool whole = p.lf >= uint32_t(V);  // uniform
+    const uint32_t j0 = whole ? min(cc * V, p.lf - uint32_t(V)) : cc * V;
+    const int drop = whole && active ? int(cc * V - j0) : 0;  // columns of the chunk before it
     const int nvalid = active ? min(V, int(p.lf - j0)) : 0;
     A acc[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) acc[v].init(p.identity);
     const uint32_t r0 = sp * p.per_split;
     const uint32_t r1 = min(p.red_count, r0 + p.per_split);
-    // the rows of this block's split; FULL: the whole tile holds whole
-    // chunks, so rows past the split's end are clamped to its last row and
-    // their values dropped, and no load sits behind a divergent branch
-    auto sweep = [&](auto full_c, auto ntm_c) {
-        constexpr bool FULL = decltype(full_c)::value;
+    // the rows of this block's split: rows past the split's end are clamped to
+    // its last row and their values dropped, so that no load sits behind a
+    // lane-dependent branch
+    auto sweep = [&](auto ntm_c) {
         constexpr int NTM = decltype(ntm_c)::value;
         for (uint32_t r = r0 + rg; r < r1; r += RG * U) {
             Reg R[U][NR][V];
@@ -500,44 +544,62 @@ __global__ __launch_bounds__(512) void reduce_cols_fast_kernel(const RedPlan p) 
             for (int u = 0; u < U; ++u) {
                 const uint32_t rr = r + RG * uint32_t(u);
                 ok[u] = rr < r1;
-                const uint32_t idx[4] = {FULL ? min(rr, r1 - 1) : rr, 0u, 0u, 0u};
-                if (FULL || ok[u]) run_spec<S, 0, V, NR, 2, FULL, NTM>(p, idx, j0, nvalid, R[u]);
+                const uint32_t idx[4] = {uint32_t(min(rr, r1 - 1)), 0u, 0u, 0u};
+                run_spec<S, 0, V, NR, 2, true, NTM>(p, idx, j0, V, R[u]);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if constexpr (FULL) {
-                    // a select, not a branch: a branch would let the compiler
-                    // sink the clamped row's load into it and wait there
+                // a select, not a branch: a branch would let the compiler
+                // sink the clamped row's load into it and wait there
 #pragma unroll
-                    for (int v = 0; v < V; ++v) {
-                        A t = acc[v];
-                        t.add(R[u][S::result_reg][v]);
-                        acc[v] = ok[u] ? t : acc[v];
-                    }
-                } else if (ok[u]) {
-#pragma unroll
-                    for (int v = 0; v < V; ++v)
-                        if (v < nvalid) acc[v].add(R[u][S::result_reg][v]);
+                for (int v = 0; v < V; ++v) {
+                    A t = acc[v];
+                    t.add(R[u][S::result_reg][v]);
+                    acc[v] = ok[u] ? t : acc[v];
                 }
             }
         }
     };
-    const bool full_tile = (tile + 1) * TW <= p.nchunks_f && p.lf == p.nchunks_f * uint32_t(V);  // uniform
     const int ntm = spec_leaves_nt<S>(p);
-    if (full_tile && ntm == 1) sweep(std::true_type{}, std::integral_constant<int, 1>{});
-    else if (full_tile && ntm == 0) sweep(std::true_type{}, std::integral_constant<int, 0>{});
-    else if (active) sweep(std::false_type{}, std::integral_constant<int, 2>{});
+    if (whole && ntm == 1) {
+        sweep(std::integral_constant<int, 1>{});
+    } else if (whole && ntm == 0) {
+        sweep(std::integral_constant<int, 0>{});
+    } else if (whole) {
+        sweep(std::integral_constant<int, 2>{});
+    } else if (active) {
+        for (uint32_t r = r0 + rg; r < r1; r += RG) {
+            Reg R[NR][V];
+            const uint32_t idx[4] = {r, 0u, 0u, 0u};
+            run_spec<S, 0, V, NR, 2>(p, idx, j0, nvalid, R);
 #pragma unroll
-    for (int v = 0; v < V; ++v) lds[threadIdx.x][v] = acc[v].lds();
+            for (int v = 0; v < V; ++v)
+                if (v < nvalid) acc[v].add(R[S::result_reg][v]);
+        }
+    }
+    if (threadIdx.x >= HB) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) lds[threadIdx.x - HB][v] = acc[v].lds();
+    }
+    __syncthreads();
+    if (threadIdx.x < HB) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            A b;
+            b.from_lds(lds[threadIdx.x][v]);
+            acc[v].merge(b);
+            lds[threadIdx.x][v] = acc[v].lds();
+        }
+    }
     __syncthreads();
     const bool merge_here = p.splits > 1 && p.counters != nullptr;  // uniform
     if (rg == 0 && active) {
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-            if (v < nvalid) {
+            if (v >= drop && v < nvalid) {
                 A a;
                 a.from_lds(lds[tl][v]);
-                for (uint32_t g = 1; g < RG; ++g) {
+                for (uint32_t g = 1; g < RG / 2; ++g) {
                     A b;
                     b.from_lds(lds[g * TW + tl][v]);
                     a.merge(b);
@@ -572,7 +634,7 @@ __global__ __launch_bounds__(512) void reduce_cols_fast_kernel(const RedPlan p) 
     if (!s_last) return;  // uniform in the block
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     const uint32_t T = uint32_t(p.combine_group);
-    const uint32_t per_pass = 512u / T;
+    const uint32_t per_pass = uint32_t(kColsBlock) / T;
     const uint32_t o0 = tile * TW * uint32_t(V);  // the tile's first output
     const uint32_t o1 = min(p.n_out, o0 + TW * uint32_t(V));
     for (uint32_t ob = o0; ob < o1; ob += per_pass) {
@@ -591,7 +653,7 @@ using KFn = void (*)(const RedPlan);
 
 struct RedKernels {
     KFn rows32, rows64, cols32, cols64;
-    KFn rows_fast1, rows_fast2, cols_fast;  // compiled fast kernels (compact plans), or null
+    KFn rows_fast1, rows_fast2, rows_fast3, cols_fast;  // compiled fast kernels (compact plans), or null
 };
 
 // specialised programs: unrolled x4, 32-bit indexing only (64-bit plans run the generic kernels)
@@ -599,7 +661,7 @@ template <int V, int NR, class S, int AK, int OP> RedKernels spec_kernels_for() 
     return RedKernels{reduce_rows_kernel<V, NR, S, false, AK, OP, 4>, nullptr,
                       reduce_cols_kernel<V, NR, S, false, AK, OP, 4>, nullptr,
                       reduce_rows_fast_kernel<V, NR, S, AK, OP, 1>, reduce_rows_fast_kernel<V, NR, S, AK, OP, 2>,
-                      reduce_cols_fast_kernel<V, NR, S, AK, OP>};
+                      reduce_rows_fast_kernel<V, NR, S, AK, OP, 3>, reduce_cols_fast_kernel<V, NR, S, AK, OP>};
 }
 
 // generic interpreter: V = 4, no unrolling
@@ -608,7 +670,7 @@ template <int AK, int OP> RedKernels dyn_kernels_for() {
                       reduce_rows_kernel<4, kMaxRegs, DynSpec, true, AK, OP, 1>,
                       reduce_cols_kernel<4, kMaxRegs, DynSpec, false, AK, OP, 1>,
                       reduce_cols_kernel<4, kMaxRegs, DynSpec, true, AK, OP, 1>,
-                      nullptr, nullptr, nullptr};
+                      nullptr, nullptr, nullptr, nullptr};
 }
 
 // generic kernels per accumulator family (defined in reduce_dyn_*.hip)

@@ -576,18 +576,22 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
     else p.per_split = uint32_t((uint64_t(p.red_count) + p.splits - 1) / p.splits);
     p.div_splits = make_fastdiv(uint32_t(p.splits));
 
-    // compact rank <= 2 form and the work split of the compiled fast kernels
-    const bool rows_ok = p.layout == RL_ROWS && p.rank <= 2 && p.n_red == 1;
+    // compact form and the work split of the compiled fast kernels
+    const bool rows3 = p.layout == RL_ROWS && p.n_red == 2 && p.n_kept <= 1;
+    const bool rows_ok = rows3 || (p.layout == RL_ROWS && p.rank <= 2 && p.n_red == 1);
     const bool cols_ok = p.layout == RL_COLS && p.rank == 2 && p.n_kept == 0;
     if (!p.index64 && (rows_ok || cols_ok) && !empty_red) {
         p.compact = 1;
+        p.f_rank = rows3 ? 3 : p.rank;
+        const int lead = p.f_rank - p.rank;  // 1: no kept dim in front
         for (int pl = 0; pl < nl; ++pl)
-            for (int k = 0; k < p.rank; ++k) p.cst[pl][k] = p.prog.leaf_gather[pl] ? 0 : int32_t(p.leaves[pl].stride[k]);
+            for (int k = 0; k < p.rank; ++k)
+                p.cst[pl][k + lead] = p.prog.leaf_gather[pl] ? 0 : int32_t(p.leaves[pl].stride[k]);
         // enough loads in flight to cover HBM latency
         const uint64_t target_waves = uint64_t(cus) * uint64_t(g_reduce_waves_per_cu);
         constexpr uint64_t kU = 4;                          // chunks (rows) in flight per lane
         if (p.layout == RL_ROWS) {
-            const uint64_t chunks = p.nchunks_f;
+            const uint64_t chunks = p.red_count;
             uint64_t g = pow2_ceil(uint32_t(std::max<uint64_t>(1, (chunks + 2 * kU - 1) / (2 * kU))));
             if (uint64_t(n_out) < target_waves) g = 64;  // few outputs: whole waves, then splits
             p.f_group = int(std::min<uint64_t>(std::max<uint64_t>(g, 1), 64));
@@ -606,23 +610,26 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
             // sum, float32 / bf16: 64 lanes 4.23 / 2.45 TB/s, 128 lanes
             // 4.19 / 2.55, 256 lanes 3.90 / 2.03; MI355X)
             const uint64_t nc = p.nchunks_f;
-            const uint64_t tw = (nc >= 128 && ((nc + 127) / 128 * 128 - nc) * 8 <= nc) ? 128 : 64;
-            const uint64_t tiles = (nc + tw - 1) / tw;
-            const uint64_t row_groups = 512 / tw;
-            // blocks of 512 threads: one per CU at the default 16 waves per CU
-            // (4.2 TB/s on a [8192, 4096] float32 column sum, 3.7 with two per CU)
+            // blocks: one per CU at the default 16 waves per CU
             const uint64_t target_blocks = std::max<uint64_t>(1, target_waves / 16 * uint64_t(g_cols_blocks_per_cu));
-            uint64_t s = (target_blocks + tiles - 1) / tiles;
-            s = std::min<uint64_t>(s, std::max<uint64_t>(1, rows / (row_groups * kU * 2)));
-            // partial results stay within about 6% of the input bytes
-            s = std::min<uint64_t>(s, std::max<uint64_t>(1, uint64_t(best) * uint64_t(g_cols_partial_mult) /
-                                                                         (uint64_t(n_out) * 16 * 16)));
+            auto splits_for = [&](uint64_t tw) {
+                const uint64_t tiles = (nc + tw - 1) / tw;
+                const uint64_t row_groups = uint64_t(kColsBlock) / tw;
+                // rounded down: a few blocks past one per CU would run after (or share a CU with) the others
+                uint64_t s = std::max<uint64_t>(1, target_blocks / tiles);
+                s = std::min<uint64_t>(s, std::max<uint64_t>(1, rows / (row_groups * kU)));
+                return std::min<uint64_t>(s, std::max<uint64_t>(1, uint64_t(best) * uint64_t(g_cols_partial_mult) /
+                                                                       (uint64_t(n_out) * 16 * 16)));
+            };
+            uint64_t tw = (nc >= 128 && ((nc + 127) / 128 * 128 - nc) * 8 <= nc) ? 128 : 64;
+            if (tw == 128 && (nc + 127) / 128 * splits_for(128) < target_blocks) tw = 64;
+            const uint64_t s = splits_for(tw);
             p.f_group = int(tw);
             p.f_splits = int(std::min<uint64_t>(s, 65535));
             p.f_per_split = uint32_t((rows + p.f_splits - 1) / p.f_splits);
         }
         while (p.f_splits > 1 && uint64_t(n_out) * uint64_t(p.f_splits) >= (uint64_t(1) << 31)) p.f_splits /= 2;
-        if (p.layout == RL_ROWS) p.f_per_split = uint32_t((uint64_t(p.nchunks_f) + p.f_splits - 1) / p.f_splits);
+        if (p.layout == RL_ROWS) p.f_per_split = uint32_t((uint64_t(p.red_count) + p.f_splits - 1) / p.f_splits);
         else p.f_per_split = uint32_t((uint64_t(p.red_count) + p.f_splits - 1) / p.f_splits);
     }
     return p;
