@@ -491,3 +491,26 @@ def test_prepared_multi_pass_and_immediate_reductions():
             ref = xt.eval(r)
             torch.cuda.synchronize()
             assert same_bits(out.to_numpy(), ref.to_numpy()), (rep, r.kind)
+
+
+@pytest.mark.parametrize("shape", [(34, 71), (1029, 575), (3, 5000), (700, 4), (1, 9), (5, 1)])
+@pytest.mark.parametrize("dtype", ["float32", "float64", "int32", "bfloat16"])
+def test_small_expressions_reduce_like_stored_ones(shape, dtype):
+    """Below the compile threshold an expression is evaluated into a temporary
+    and reduced like an array: eager, prepared and on the stored values the
+    results are the same bits, for every kind and axis."""
+    rng = np.random.default_rng(sum(shape))
+    h = rng.integers(-50, 50, shape).astype("int32") if dtype == "int32" else rng.normal(size=shape).astype(
+        "float32" if dtype == "bfloat16" else dtype)
+    x = xt.from_numpy(h, dtype)
+    e = x * x - x
+    stored = xt.eval(e)
+    for kind in ("sum", "mean", "amax", "amin", "norm_l2", "variance"):
+        for axes in ([0], [1], None):
+            f = getattr(xt, kind)
+            got = xt.eval(f(e, axes))
+            want = xt.eval(f(stored, axes)).to_numpy()
+            assert same_bits(got.to_numpy(), want), (kind, axes)
+            out = xt.empty(got.shape, got.dtype)
+            xt.plan(out, f(e, axes)).run()
+            assert same_bits(out.to_numpy(), want), (kind, axes)

@@ -33,6 +33,10 @@ template <int OP> struct Acc<AK_F32C, OP> {
         s = t;
         c = c + o.c + err;
     }
+    // `o` if k.  Member by member: a conditional of two structs selects between
+    // their addresses, which kept a float64 pair in scratch memory (the float64
+    // channel mean of [32, 256, 28, 28]: 36.3 us, 16.0 us this way).
+    __device__ void pick(bool k, const Acc& o) { s = k ? o.s : s; c = k ? o.c : c; }
     __device__ Acc shfl_xor(int m) const { Acc r; r.s = __shfl_xor(s, m); r.c = __shfl_xor(c, m); return r; }
     __device__ Acc shfl_up(int d) const { Acc r; r.s = __shfl_up(s, d); r.c = __shfl_up(c, d); return r; }
     __device__ Acc shfl_idx(int src) const { Acc r; r.s = __shfl(s, src); r.c = __shfl(c, src); return r; }
@@ -65,6 +69,7 @@ template <int OP> struct Acc<AK_F64C, OP> {
         s = t;
         c = c + o.c + err;
     }
+    __device__ void pick(bool k, const Acc& o) { s = k ? o.s : s; c = k ? o.c : c; }
     __device__ Acc shfl_xor(int m) const { Acc r; r.s = __shfl_xor(s, m); r.c = __shfl_xor(c, m); return r; }
     __device__ Acc shfl_up(int d) const { Acc r; r.s = __shfl_up(s, d); r.c = __shfl_up(c, d); return r; }
     __device__ Acc shfl_idx(int src) const { Acc r; r.s = __shfl(s, src); r.c = __shfl(c, src); return r; }
@@ -121,6 +126,7 @@ template <int AK, int OP> struct Acc {
     __device__ void init(uint64_t id) { v = reg_get<T>(id); }
     __device__ void add(Reg x) { v = combine(v, reg_get<T>(x)); }
     __device__ void merge(const Acc& o) { v = combine(v, o.v); }
+    __device__ void pick(bool k, const Acc& o) { v = k ? o.v : v; }
     __device__ Acc shfl_xor(int m) const { Acc r; r.v = __shfl_xor(v, m); return r; }
     __device__ Acc shfl_up(int d) const { Acc r; r.v = __shfl_up(v, d); return r; }
     __device__ Acc shfl_idx(int src) const { Acc r; r.v = __shfl(v, src); return r; }

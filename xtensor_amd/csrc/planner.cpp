@@ -548,11 +548,25 @@ Program lower(const xg_expr* e, const ExprInfo& info, int final_dt, int map) {
 }
 
 int choose_vector_width(const xg_expr* e, const xg_tensor* out) {
-    // each lane moves 16 bytes of the widest operand per access, so a wave's
-    // access is 1 KiB of consecutive memory
-    int w = out ? dtype_size(out->dtype) : 1;
-    for (int l = 0; e && l < e->n_leaves; ++l) w = std::max(w, dtype_size(e->leaves[l].dtype));
-    return std::max(2, std::min(16, 16 / w));
+    // each lane moves 16 bytes of the widest streamed operand per access, so a
+    // wave's access is 1 KiB of consecutive memory.  Operands a sixteenth of
+    // the largest or smaller (a row, a value per channel) come from the caches
+    // and do not narrow the others: a float32 batch less its float64 channel
+    // means is read 16 bytes at a time, not 8.
+    auto elements = [](const xg_tensor& t) {
+        double n = 1;
+        for (int k = 0; k < t.ndim && k < XG_MAX_RANK; ++k) n *= double(std::max<int64_t>(t.shape[k], 0));
+        return n;
+    };
+    double most = out ? elements(*out) : 0;
+    for (int l = 0; e && l < e->n_leaves; ++l) most = std::max(most, elements(e->leaves[l]));
+    int w = out ? dtype_size(out->dtype) : 1, any = w;
+    for (int l = 0; e && l < e->n_leaves; ++l) {
+        const int esz = dtype_size(e->leaves[l].dtype);
+        any = std::max(any, esz);
+        if (elements(e->leaves[l]) * 16 > most) w = std::max(w, esz);
+    }
+    return std::max(2, std::min(16 / w, 64 / any));
 }
 
 // ------------------------------------------------------------------ assign plan

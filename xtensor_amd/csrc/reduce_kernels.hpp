@@ -392,6 +392,14 @@ template <int NR, int V, bool COLS> constexpr int fast_unroll() {
     return NR * V <= 8 ? 4 : (NR * V <= 16 ? 2 : 1);
 }
 
+// Between the loads of U chunks and the folding of their values: arithmetic
+// may be scheduled across, loads not.  Without it the scheduler, saving
+// registers, puts each chunk's loads right before their use and the chunks
+// wait one after the other (a variance's deviations over [64, 256, 28, 28]
+// float32 issued its four chunks in four waits; the four loads now go out
+// together).
+__device__ __forceinline__ void loads_issued() { __builtin_amdgcn_sched_barrier(0x7); }
+
 // Ragged rows (lf no multiple of V): the last chunk of a row is read as the
 // row's last V elements and the leading ones, which the chunk before it holds,
 // are dropped with a select, so that no load sits behind a lane-dependent
@@ -450,6 +458,7 @@ __global__ __launch_bounds__(256) void reduce_rows_fast_kernel(const RedPlan p) 
                 }
                 run_spec<S, 0, V, NR, RANK, true, NTM>(p, idx, j0, V, R[u]);
             }
+            loads_issued();
 #pragma unroll
             for (int u = 0; u < U; ++u) {  // selects, not branches (see the cols kernel)
                 if constexpr (RAGGED) {
@@ -457,13 +466,13 @@ __global__ __launch_bounds__(256) void reduce_rows_fast_kernel(const RedPlan p) 
                     for (int v = 0; v < V; ++v) {
                         A t = acc;
                         t.add(R[u][S::result_reg][v]);
-                        acc = ok[u] && uint32_t(v) >= drop[u] ? t : acc;
+                        acc.pick(ok[u] && uint32_t(v) >= drop[u], t);
                     }
                 } else {
                     A t = acc;
 #pragma unroll
                     for (int v = 0; v < V; ++v) t.add(R[u][S::result_reg][v]);
-                    acc = ok[u] ? t : acc;
+                    acc.pick(ok[u], t);
                 }
             }
         }
@@ -547,6 +556,7 @@ __global__ __launch_bounds__(kColsBlock) void reduce_cols_fast_kernel(const RedP
                 const uint32_t idx[4] = {uint32_t(min(rr, r1 - 1)), 0u, 0u, 0u};
                 run_spec<S, 0, V, NR, 2, true, NTM>(p, idx, j0, V, R[u]);
             }
+            loads_issued();
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 // a select, not a branch: a branch would let the compiler
@@ -555,7 +565,7 @@ __global__ __launch_bounds__(kColsBlock) void reduce_cols_fast_kernel(const RedP
                 for (int v = 0; v < V; ++v) {
                     A t = acc[v];
                     t.add(R[u][S::result_reg][v]);
-                    acc[v] = ok[u] ? t : acc[v];
+                    acc[v].pick(ok[u], t);
                 }
             }
         }

@@ -629,8 +629,18 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
             p.f_per_split = uint32_t((rows + p.f_splits - 1) / p.f_splits);
         }
         while (p.f_splits > 1 && uint64_t(n_out) * uint64_t(p.f_splits) >= (uint64_t(1) << 31)) p.f_splits /= 2;
-        if (p.layout == RL_ROWS) p.f_per_split = uint32_t((uint64_t(p.red_count) + p.f_splits - 1) / p.f_splits);
-        else p.f_per_split = uint32_t((uint64_t(p.red_count) + p.f_splits - 1) / p.f_splits);
+        p.f_per_split = uint32_t((uint64_t(p.red_count) + p.f_splits - 1) / p.f_splits);
+        if (p.layout == RL_ROWS && p.f_splits > 1) {
+            // whole rounds of kU chunks a lane: a split of 12.25 chunks a lane
+            // costs four rounds, the last one mostly dropped values
+            const uint64_t round = uint64_t(p.f_group) * kU;
+            const uint64_t k = std::max<uint64_t>(1, (p.f_per_split + round / 2) / round);
+            const uint64_t s = (uint64_t(p.red_count) + k * round - 1) / (k * round);
+            if (s <= 65535 && s * n_out < (uint64_t(1) << 31)) {
+                p.f_per_split = uint32_t(k * round);
+                p.f_splits = int(s);
+            }
+        }
     }
     return p;
 }

@@ -124,6 +124,13 @@ Shape leaf_only(Builder& b, int dt, Shape s) {
     return s;
 }
 
+Shape deviation(Builder& b, int dt, Shape mean) {
+    int x = b.leaf(Builder::tensor(dt, {512, 2048}));
+    int m = b.leaf(Builder::tensor(XG_FLOAT64, mean));
+    b.bin(XG_OP_MINUS, x, m);
+    return Shape{512, 2048};
+}
+
 const std::vector<RSpecDef>& rspec_defs() {
     static const std::vector<RSpecDef> defs = {
         {"sum_f32", XG_RED_SUM, {1}, [](Builder& b) { return leaf_only(b, XG_FLOAT32, {8192, 4096}); }},
@@ -149,6 +156,14 @@ const std::vector<RSpecDef>& rspec_defs() {
              b.un(XG_OP_EXP, b.bin(XG_OP_MINUS, x, m));
              return Shape{512, 2048};
          }},
+        // the squared deviations of a variance: x less a float64 mean per row
+        // (per channel), and per column
+        {"dev_sq_rows_f32", XG_RED_VARIANCE, {1}, [](Builder& b) { return deviation(b, XG_FLOAT32, {512, 1}); }},
+        {"dev_sq_rows_bf16", XG_RED_VARIANCE, {1}, [](Builder& b) { return deviation(b, XG_BFLOAT16, {512, 1}); }},
+        {"dev_sq_rows_f64", XG_RED_VARIANCE, {1}, [](Builder& b) { return deviation(b, XG_FLOAT64, {512, 1}); }},
+        {"dev_sq_cols_f32", XG_RED_VARIANCE, {0}, [](Builder& b) { return deviation(b, XG_FLOAT32, {1, 2048}); }},
+        {"dev_sq_cols_bf16", XG_RED_VARIANCE, {0}, [](Builder& b) { return deviation(b, XG_BFLOAT16, {1, 2048}); }},
+        {"dev_sq_cols_f64", XG_RED_VARIANCE, {0}, [](Builder& b) { return deviation(b, XG_FLOAT64, {1, 2048}); }},
     };
     return defs;
 }

@@ -33,6 +33,7 @@ struct Arena {
     size_t cap = 0;
     size_t used = 0;
     uint32_t* counters = nullptr;  // column reductions' arrival counters, or none
+    bool eval_first = false;  // small expressions may be evaluated into a temporary of the block
     // `bytes` (256-byte aligned) from the block; nullptr for 0 bytes
     char* take(size_t bytes);
 };

@@ -107,37 +107,39 @@ constexpr int64_t kNtMinBytes = int64_t(64) << 20;
 
 // Division by a run-time constant with a precomputed multiplier
 // (Granlund & Montgomery, "Division by invariant integers using
-// multiplication", PLDI 1994, round-up variant for 32-bit unsigned n < 2^31).
+// multiplication", PLDI 1994, round-up variant for 32-bit unsigned n < 2^31):
+// q = (t + ((n - t) >> pre)) >> post with t = mulhi(n, mul).  No branch, also
+// not for d = 1 (pre = post = 0, t = 0): a branch between the addresses of
+// several loads keeps the compiler from issuing them together.
 struct FastDiv {
     uint32_t d;
     uint32_t mul;
-    uint32_t shift;
-    uint32_t pad_;
+    uint32_t pre;
+    uint32_t post;
 };
 
 XG_HD inline FastDiv make_fastdiv(uint32_t d) {
-    FastDiv f{d, 0, 0, 0};
-    if (d <= 1) { f.mul = 0; f.shift = 0; return f; }
+    FastDiv f{d, 1, 0, 0};
+    if (d <= 1) return f;
     uint32_t l = 0;
     while ((1ull << l) < d) ++l;  // l = ceil(log2 d)
     uint64_t m = ((1ull << 32) * ((1ull << l) - d)) / d + 1;
     f.mul = uint32_t(m);
-    f.shift = l;
+    f.pre = 1;
+    f.post = l - 1;
     return f;
 }
 
 #if defined(__HIPCC__)
 __device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv& f) {
-    if (f.d == 1) return n;
-    uint32_t t = __umulhi(n, f.mul);
-    return (t + ((n - t) >> 1)) >> (f.shift - 1);
+    const uint32_t t = __umulhi(n, f.mul);
+    return (t + ((n - t) >> f.pre)) >> f.post;
 }
 #endif
 
 XG_HD inline uint32_t fastdiv_host(uint32_t n, const FastDiv& f) {
-    if (f.d == 1) return n;
-    uint32_t t = uint32_t((uint64_t(n) * f.mul) >> 32);
-    return (t + ((n - t) >> 1)) >> (f.shift - 1);
+    const uint32_t t = uint32_t((uint64_t(n) * f.mul) >> 32);
+    return (t + ((n - t) >> f.pre)) >> f.post;
 }
 
 // ---------------------------------------------------------------- programs
