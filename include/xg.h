@@ -352,6 +352,17 @@ xg_status xg_assign_indexed(const xg_expr* values, const xg_expr* offsets, const
  * device, no host copy of the condition. */
 xg_status xg_argwhere(const xg_expr* cond, int32_t column_major, const xg_tensor* out, xg_stream_t stream);
 
+/* The same in two steps, for callers that do not know count: the condition is
+ * evaluated once.  xg_argwhere_buffer gives the bytes of a device buffer for n
+ * elements and where in it the count (int64) will be; xg_argwhere_mark fills
+ * the caller's buffer (16-byte aligned); after reading the count back the
+ * caller allocates out and xg_argwhere_list writes the rows.  The buffer is
+ * the caller's and holds everything between the steps. */
+xg_status xg_argwhere_buffer(int64_t n, size_t* bytes, size_t* total_at);
+xg_status xg_argwhere_mark(const xg_expr* cond, int32_t column_major, void* buffer, xg_stream_t stream);
+xg_status xg_argwhere_list(const xg_expr* cond, int32_t column_major, const void* buffer, const xg_tensor* out,
+                           xg_stream_t stream);
+
 /* ---- .npy files to and from device memory (io/xnpy.hpp) ------------------
  * Header of an .npy file: dtype, shape and order (xt::detail::load_npy_file's
  * header parse, io/xnpy.hpp:236-393, 646-673).  A type string without a

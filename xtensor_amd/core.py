@@ -1043,20 +1043,29 @@ def count_nonzero(e) -> int:
 def argwhere(cond, layout="row_major") -> DeviceArray:
     """xt::argwhere<L> (core/xoperation.hpp:893-930): int64 [count, ndim]
     multi-indices of the true elements in row-major (or column-major)
-    traversal order, listed on the device (xg_argwhere: a scan of the flags
-    and one compaction kernel); only the count is read back, to size the
+    traversal order, listed on the device: the condition is evaluated once,
+    its true elements counted, and only the count is read back, to size the
     result."""
     c = _wrap(cond)
     if layout not in ("row_major", "column_major"):
         raise ValueError("layout is 'row_major' or 'column_major'")
-    _, shp = expr_info(c)
-    n = count_nonzero(c)
-    out = empty((n, len(shp)), "int64")
-    if n:
-        _require_device(_leaves(c) + [out])
-        s = serialize(c, reducer_fn=_eval_reducer)
-        t = out.to_abi()
-        _check(A.lib().xg_argwhere(s.ptr(), 1 if layout == "column_major" else 0, C.byref(t), _stream()))
+    p = _pack(c, _eval_reducer)
+    _, shp = _info(p.info())
+    n = math.prod(shp)
+    if not shp or n == 0:
+        if count_nonzero(c):
+            raise ValueError("argwhere of a 0-d expression")
+        return _empty((0, len(shp)), A.INT64)
+    torch = _torch()
+    nbytes, at = C.c_size_t(), C.c_size_t()
+    _check(A.lib().xg_argwhere_buffer(n, C.byref(nbytes), C.byref(at)))
+    buf = torch.empty(nbytes.value, dtype=torch.uint8, device="cuda")
+    order, ptr, stream = int(layout == "column_major"), buf.data_ptr(), _raw_stream()
+    _check(p.argwhere_mark(order, ptr, stream))
+    rows = int(buf[at.value:at.value + 8].view(torch.int64).item())
+    out = _empty((rows, len(shp)), A.INT64)
+    if rows:
+        _check(p.argwhere_list(order, ptr, out, stream))
     return out
 
 

@@ -475,19 +475,39 @@ PyObject* m_scan(PyObject* self, PyObject* const* a, Py_ssize_t n) {  // (op, dt
     return PyLong_FromLong(r);
 }
 
-PyObject* m_argwhere(PyObject* self, PyObject* const* a, Py_ssize_t n) {  // (order, out, stream)
+PyObject* m_argwhere_mark(PyObject* self, PyObject* const* a, Py_ssize_t n) {  // (order, buffer, stream)
+    Packed* p = reinterpret_cast<Packed*>(self);
+    long long order = 0;
+    if (n != 3) {
+        PyErr_SetString(PyExc_TypeError, "argwhere_mark(order, buffer, stream)");
+        return nullptr;
+    }
+    if (!int_of(a[0], &order) || !on_gpu(p->cuda)) return nullptr;
+    void* buf = PyLong_AsVoidPtr(a[1]);
+    xg_stream_t st = reinterpret_cast<xg_stream_t>(PyLong_AsVoidPtr(a[2]));
+    if (PyErr_Occurred()) return nullptr;
+    int r;
+    Py_BEGIN_ALLOW_THREADS
+    r = xg_argwhere_mark(&p->e, int32_t(order), buf, st);
+    Py_END_ALLOW_THREADS
+    return PyLong_FromLong(r);
+}
+
+PyObject* m_argwhere_list(PyObject* self, PyObject* const* a, Py_ssize_t n) {  // (order, buffer, out, stream)
     Packed* p = reinterpret_cast<Packed*>(self);
     xg_tensor t;
     xg_stream_t st;
     long long order = 0;
-    if (n != 3) {
-        PyErr_SetString(PyExc_TypeError, "argwhere(order, out, stream)");
+    if (n != 4) {
+        PyErr_SetString(PyExc_TypeError, "argwhere_list(order, buffer, out, stream)");
         return nullptr;
     }
-    if (!int_of(a[0], &order) || !target(p, a[1], a[2], &t, &st)) return nullptr;
+    if (!int_of(a[0], &order) || !target(p, a[2], a[3], &t, &st)) return nullptr;
+    void* buf = PyLong_AsVoidPtr(a[1]);
+    if (PyErr_Occurred()) return nullptr;
     int r;
     Py_BEGIN_ALLOW_THREADS
-    r = xg_argwhere(&p->e, int32_t(order), &t, st);
+    r = xg_argwhere_list(&p->e, int32_t(order), buf, &t, st);
     Py_END_ALLOW_THREADS
     return PyLong_FromLong(r);
 }
@@ -501,7 +521,8 @@ PyMethodDef packed_methods[] = {
     {"assign", XG_FAST(m_assign), METH_FASTCALL, "xg_assign(out, stream)"},
     {"reduce", XG_FAST(m_reduce), METH_FASTCALL, "xg_reduce(reducer, out, stream)"},
     {"scan", XG_FAST(m_scan), METH_FASTCALL, "xg_scan(op, dtype, axis, out, stream)"},
-    {"argwhere", XG_FAST(m_argwhere), METH_FASTCALL, "xg_argwhere(order, out, stream)"},
+    {"argwhere_mark", XG_FAST(m_argwhere_mark), METH_FASTCALL, "xg_argwhere_mark(order, buffer, stream)"},
+    {"argwhere_list", XG_FAST(m_argwhere_list), METH_FASTCALL, "xg_argwhere_list(order, buffer, out, stream)"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyTypeObject packed_type = [] {

@@ -255,6 +255,12 @@ void assign_launch(const xg_expr* e, const xg_tensor* out, hipStream_t st, const
     check_hip(launch_ew(p, V, device_cus(), st, used), "elementwise launch");
 }
 
+}  // namespace
+
+void xg::assign_any(const xg_expr* e, const xg_tensor* out, hipStream_t st) { assign_launch(e, out, st, nullptr); }
+
+namespace {
+
 // Launch a planned reduction with its split partials from the arena.
 void run_reduce(RedPlan& p, int V, hipStream_t st, Arena& a, const char** used) {
     p.partials = a.take(reduce_workspace_bytes(p));

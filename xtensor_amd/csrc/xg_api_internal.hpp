@@ -38,6 +38,9 @@ struct Arena {
     char* take(size_t bytes);
 };
 
+// out = e by one plan or in pieces (what xg_assign runs)
+void assign_any(const xg_expr* e, const xg_tensor* out, hipStream_t st);
+
 // Where the block of a call comes from: `get(bytes)` returns at least
 // `bytes` of device memory usable in stream order on the call's stream.
 using BlockSource = char* (*)(size_t bytes, hipStream_t stream, void* ctx);
