@@ -312,3 +312,38 @@ def test_full_uneven_batch_4096_vs_fp64():
     sync()
     assert same_bits(first, xout.to_numpy())
     assert b.info()["elements"] == sum(r * c for r, c in shapes)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("op", ["softmax", "sum", "amax"])
+def test_narrow_rows_with_and_without_a_queue(op, dtype):
+    """Rows of at most one element a lane, at the edges of the 4 .. 64 lane
+    groups, in row counts around a wave's rows; scheduled by the host alone,
+    partly and wholly from the queue, launched and as a graph.  amax is exact;
+    a sum of at most 64 terms, accumulated in at least float64 or compensated
+    float32, is off by half an ulp of the result's rounding plus second-order
+    terms: 2 eps |x|_1 bounds it.  softmax as at the top."""
+    shapes = [(r, c) for c in (1, 3, 4, 5, 8, 9, 16, 17, 32, 33, 63, 64) for r in (1, 2, 15, 16, 17, 65)]
+    eps = np.finfo(dtype).eps
+    xs, dx, outs = make(shapes, dtype, op=op)
+    first = None
+    for dyn in (0, 10, 100):
+        b = Batch(op, dx, outs)
+        b.tuning = {"block": 256, "blocks_per_cu": 5, "task_elems": 512, "dyn_percent": dyn}
+        for run in (b.launch, b.launch, b.execute, b.execute):
+            for o in outs:
+                o.storage.zero_()
+            run()
+            sync()
+            got = [o.to_numpy() for o in outs]
+            if first is None:
+                first = got
+            assert all(same_bits(g, f) for g, f in zip(got, first)), (dyn, run)
+    for x, g in zip(xs, first):
+        x64 = x.astype(np.float64)
+        if op == "amax":
+            assert np.array_equal(g, x.max(axis=1))
+        elif op == "sum":
+            assert np.all(np.abs(g - x64.sum(axis=1)) <= 2 * eps * np.abs(x64).sum(axis=1))
+        else:
+            assert rel_err(g, softmax64(x)) <= (1e-6 if dtype == np.float32 else 1e-13)

@@ -13,7 +13,7 @@
 // row — never on the batch around it or on the schedule.
 //
 // Host side: task split and schedule (longest task first onto the least
-// loaded wave), a two-node HIP graph (queue reset, kernel) per batch, and an
+// loaded wave), a HIP graph (queue reset if there is a queue, kernel) per batch, and an
 // autotuner over task size, launch shape and queue share whose choice is
 // cached per shape class.
 #include <hip/hip_runtime.h>
@@ -166,10 +166,18 @@ constexpr uint32_t kOffNone = 0x80000000u;  // an offset past every resource
 // x[sl + k * LPR], k < NE.  One buffer resource spans a row group (its
 // first row to the end of its last row inside the task), so all RB * NE
 // loads go out back to back, unmasked.
+// LPR = 64 for rows of more than one element a lane; rows of one element a lane
+// (NE = 1) share one form, LPR = 0, with their 4 .. 64 lanes as the
+// wave-uniform `lpr_rt`.  One form for them keeps the kernel's instructions at
+// 60 KB: with one per lane count they were 92 KB, more than the 64 KB cache two
+// CUs share, and a batch waited for its code (8 instances, one trip each: 55.9
+// us a launch, 14.7 now; 1024 instances 99.1 -> 47.6 with the schedule below).
 template <class T, int OP, int LPR, int NE, int RB>
-__device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, int rb, int sub, int sl) {
+__device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, int rb, int sub, int sl, int lpr_rt) {
     using Tr = BTraits<T>;
-    constexpr int PER = 64 / LPR;
+    static_assert(LPR == 64 || (LPR == 0 && NE == 1), "lane counts below a wave are run-time values");
+    const int lpr = LPR ? LPR : lpr_rt;
+    const int PER = LPR ? 1 : 64 >> (__ffs(lpr_rt) - 1);
     constexpr uint32_t E = sizeof(T);
     const int cols = it.cols;
     T v[RB][NE];
@@ -184,15 +192,15 @@ __device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, 
         const uint32_t loff = (uint32_t(sub) * uint32_t(it.in_rs) + uint32_t(sl)) * E;
 #pragma unroll
         for (int k = 0; k < NE; ++k) {
-            // element sl + k * LPR.  For NE >= 2 the class guarantees
-            // cols > (NE / 2) * LPR, so the first half is always inside the
+            // element sl + k * lpr.  For NE >= 2 the class guarantees
+            // cols > (NE / 2) * lpr, so the first half is always inside the
             // row.  (Skipping chunks wholly past the row end with a uniform
             // branch was measured slower: it splits the batch of loads.)
             // The lane-dependent part stays on the left of the comparison so
             // that no per-k lane value is kept live.
-            const bool in = (NE >= 2 && k < NE / 2) || sl < cols - k * LPR;
-            const T x = bload<T>(rin[g], loff + uint32_t(k * LPR) * E);
-            if constexpr (OP == BO_SUM) v[g][k] = (PER == 1 || in) ? x : T(0);
+            const bool in = (NE >= 2 && k < NE / 2) || sl < cols - k * lpr;
+            const T x = bload<T>(rin[g], loff + uint32_t(k * lpr) * E);
+            if constexpr (OP == BO_SUM) v[g][k] = (LPR == 64 || in) ? x : T(0);
             else v[g][k] = in ? x : Tr::lowest();
         }
     }
@@ -205,7 +213,7 @@ __device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, 
             for (int k = 1; k < NE; ++k) m[g] = OP == BO_SOFTMAX ? max_num(m[g], v[g][k]) : fmax_x(m[g], v[g][k]);
         }
 #pragma unroll
-        for (int g = 0; g < RB; ++g) m[g] = sub_max(m[g], LPR);
+        for (int g = 0; g < RB; ++g) m[g] = sub_max(m[g], lpr);
     }
     if constexpr (OP == BO_MAX) {
 #pragma unroll
@@ -221,14 +229,14 @@ __device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, 
 #pragma unroll
             for (int k = 0; k < NE; ++k) {
                 if constexpr (OP == BO_SOFTMAX) {
-                    const bool in = (NE >= 2 && k < NE / 2) || sl < cols - k * LPR;
+                    const bool in = (NE >= 2 && k < NE / 2) || sl < cols - k * lpr;
                     v[g][k] = in ? exp_shifted(v[g][k], m[g]) : T(0);
                 }
                 s[g].add(Tr::reg(v[g][k]));
             }
         }
 #pragma unroll
-        for (int g = 0; g < RB; ++g) s[g] = sub_combine(s[g], LPR);
+        for (int g = 0; g < RB; ++g) s[g] = sub_combine(s[g], lpr);
 #pragma unroll
         for (int g = 0; g < RB; ++g) {
             const int r = rb + g * PER + sub;
@@ -245,7 +253,7 @@ __device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, 
                 const uint32_t loff = (uint32_t(sub) * uint32_t(it.out_rs) + uint32_t(sl)) * E;
 #pragma unroll
                 for (int k = 0; k < NE; ++k) {
-                    const uint32_t off = (sub < nvalid && sl < cols - k * LPR) ? loff + uint32_t(k * LPR) * E : kOffNone;
+                    const uint32_t off = (sub < nvalid && sl < cols - k * lpr) ? loff + uint32_t(k * lpr) * E : kOffNone;
                     bstore<T>(ro, off, div_by(v[g][k], sum, rcp));
                 }
             }
@@ -284,15 +292,16 @@ __device__ __forceinline__ void row_stream(const BItem& it, int row, bool valid,
 
 template <class T, int OP, int LPR, int NE>
 __device__ __forceinline__ void rows_loop(const BItem& it, int nrows, int row0, int lane) {
-    constexpr int PER = 64 / LPR;
     constexpr int RB = batch_rows_at_once(NE, int(sizeof(T)));
-    for (int rb = 0; rb < nrows; rb += PER * RB) {
+    const int shift = LPR == 64 ? 6 : __ffs(it.lpr) - 1;
+    const int step = (64 >> shift) * RB;
+    for (int rb = 0; rb < nrows; rb += step) {
         // The lane number is made opaque once per iteration: otherwise the
         // compiler hoists every per-element lane offset of every variant to
         // the kernel entry, where they stay live (and spill) for its whole run.
         int l = lane;
         asm volatile("" : "+v"(l));
-        rows_regs<T, OP, LPR, NE, RB>(it, nrows, row0, rb, l / LPR, l % LPR);
+        rows_regs<T, OP, LPR, NE, RB>(it, nrows, row0, rb, l >> shift, l & ((1 << shift) - 1), 1 << shift);
     }
 }
 
@@ -312,7 +321,8 @@ __global__ __launch_bounds__(256, 5) void batch_rows_kernel(const BatchArgs a) {
     uint32_t t = a.wbeg[w];
     uint32_t tend = a.wbeg[w + 1];
     for (;; ++t) {
-        if (t >= tend) {  // own list done: take from the shared queue
+        if (t >= tend) {  // own list done: take from the shared queue, if there is one
+            if (a.dyn_begin >= a.ntasks) break;
             uint32_t q = 0;
             if (lane == 0) q = atomicAdd(a.counter, 1u);
             t = a.dyn_begin + __builtin_amdgcn_readlane(q, 0);  // wave-uniform from here on
@@ -325,11 +335,7 @@ __global__ __launch_bounds__(256, 5) void batch_rows_kernel(const BatchArgs a) {
         const int row0 = task.row0;
         const int ne = batch_ne_class(it.cols, it.lpr, int(sizeof(T)));  // the same for the whole task
         if (it.cols == 0) rows_empty<T, OP>(it, nrows, row0, lane);
-        else if (it.lpr == 4) rows_loop<T, OP, 4, 1>(it, nrows, row0, lane);
-        else if (it.lpr == 8) rows_loop<T, OP, 8, 1>(it, nrows, row0, lane);
-        else if (it.lpr == 16) rows_loop<T, OP, 16, 1>(it, nrows, row0, lane);
-        else if (it.lpr == 32) rows_loop<T, OP, 32, 1>(it, nrows, row0, lane);
-        else if (ne == 1) rows_loop<T, OP, 64, 1>(it, nrows, row0, lane);
+        else if (ne == 1) rows_loop<T, OP, 0, 1>(it, nrows, row0, lane);  // 4 to 64 lanes a row
         else if (ne == 2) rows_loop<T, OP, 64, 2>(it, nrows, row0, lane);
         else if (ne == 4) rows_loop<T, OP, 64, 4>(it, nrows, row0, lane);
         else if (ne == 8) rows_loop<T, OP, 64, 8>(it, nrows, row0, lane);
@@ -438,7 +444,11 @@ std::map<ClassKey, xg_batch_tuning> g_tune_cache;
 
 int ilog2(double x) { return x < 1.0 ? 0 : int(std::floor(std::log2(x))); }
 
-xg_batch_tuning default_tuning() { return xg_batch_tuning{256, 4, 2048, 10}; }
+// Small tasks spread a small batch over the waves, and a purely host-balanced
+// schedule spares every wave its visit to the queue's one counter (float32
+// softmax, default {256, 4, 2048, 10} -> this: 64 instances 68.0 -> 21.5 us,
+// 357 71.6 -> 34.8, 1024 99.1 -> 47.6, 4096 272 -> 223).
+xg_batch_tuning default_tuning() { return xg_batch_tuning{256, 5, 512, 0}; }
 
 void check_tuning(const xg_batch_tuning& t) {
     if (t.block < 64 || t.block > 256 || t.block % 64 != 0)
@@ -573,16 +583,22 @@ struct xg_batch_s {
         if (!h.empty()) check_hip(hipMemcpy(dptr, h.data(), h.size() * sizeof(V), hipMemcpyHostToDevice), "hipMemcpy");
     }
 
+    // A schedule without a queue needs no reset; a batch without tasks keeps it
+    // as the one node of its graph.
+    bool resets() const { return tasks.empty() || dyn_begin < tasks.size(); }
+
     void enqueue(hipStream_t stream) const {
         BatchKernel k = batch_kernel_for(op, dtype);
-        hipLaunchKernelGGL(batch_reset_kernel, dim3(1), dim3(64), 0, stream, d_counter);
-        check_hip(hipGetLastError(), "batch reset launch");
+        if (resets()) {
+            hipLaunchKernelGGL(batch_reset_kernel, dim3(1), dim3(64), 0, stream, d_counter);
+            check_hip(hipGetLastError(), "batch reset launch");
+        }
         if (tasks.empty()) return;
         hipLaunchKernelGGL(k, dim3(grid_blocks()), dim3(tune.block), 0, stream, args());
         check_hip(hipGetLastError(), "batch kernel launch");
     }
 
-    // two kernel nodes: queue reset -> persistent kernel
+    // kernel nodes: queue reset (if there is a queue) -> persistent kernel
     void build_graph() {
         drop_graph();
         check_hip(hipGraphCreate(&graph, 0), "hipGraphCreate");
@@ -596,7 +612,7 @@ struct xg_batch_s {
         rp.kernelParams = reset_args;
         rp.extra = nullptr;
         hipGraphNode_t n_reset = nullptr;
-        check_hip(hipGraphAddKernelNode(&n_reset, graph, nullptr, 0, &rp), "hipGraphAddKernelNode");
+        if (resets()) check_hip(hipGraphAddKernelNode(&n_reset, graph, nullptr, 0, &rp), "hipGraphAddKernelNode");
         if (!tasks.empty()) {
             BatchArgs a = args();
             void* kargs[] = {&a};
@@ -608,7 +624,7 @@ struct xg_batch_s {
             kp.kernelParams = kargs;
             kp.extra = nullptr;
             hipGraphNode_t n_k = nullptr;
-            check_hip(hipGraphAddKernelNode(&n_k, graph, &n_reset, 1, &kp), "hipGraphAddKernelNode");
+            check_hip(hipGraphAddKernelNode(&n_k, graph, n_reset ? &n_reset : nullptr, n_reset ? 1 : 0, &kp), "hipGraphAddKernelNode");
         }
         check_hip(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate");
     }
@@ -698,7 +714,7 @@ xg_status xg_batch_autotune(xg_batch_t b, xg_stream_t stream) {
         // assumes every wave of the grid is resident from the start.
         static const int kBlocks[] = {128, 256};
         static const int kWavesPerCu[] = {8, 12, 16, 20, 24, 32};
-        static const int kElems[] = {1024, 2048, 4096, 8192};
+        static const int kElems[] = {512, 1024, 2048, 4096, 8192};
         static const int kDyn[] = {0, 10, 30};
         hipEvent_t e0, e1;
         check_hip(hipEventCreate(&e0), "hipEventCreate");
