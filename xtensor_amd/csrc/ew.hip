@@ -157,6 +157,10 @@ hipError_t launch_ew_multi(int spec_index, int rank, const CompactPlan* d_plans,
 hipError_t launch_ew(const EwPlan& p, int V, int cus, hipStream_t stream, const char** used) {
     if (p.units == 0) return hipSuccess;
     dim3 grid(ew_grid(p.units, cus)), block(256);
+    if (!force_dynamic() && ew_is_transpose(p)) {
+        if (used) *used = "transpose";
+        return launch_ew_transpose(p, stream);
+    }
     if (!force_dynamic() && p.compact) {
         SpecKey k = spec_key(p);
         for (auto& s : spec_table()) {

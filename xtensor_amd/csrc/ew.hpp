@@ -13,6 +13,10 @@ namespace xg {
 hipError_t launch_ew(const EwPlan& p, int V, int cus, hipStream_t stream, const char** used);
 // The same by the generic interpreter (V = ew_interp_width(p)).
 hipError_t launch_ew_interp(const EwPlan& p, int V, dim3 grid, hipStream_t stream);
+// A copy whose leaf and output are contiguous along different dimensions, and
+// its launch by tiles.
+bool ew_is_transpose(const EwPlan& p);
+hipError_t launch_ew_transpose(const EwPlan& p, hipStream_t stream);
 #endif
 
 // Name of the compiled specialisation that matches the plan, or nullptr.
