@@ -6,9 +6,11 @@
 // travels several times.  Here a workgroup copies a 64 x 64 tile through LDS:
 // 16-byte loads along the leaf's contiguous dimension, 16-byte stores along
 // the output's, each line touched by one workgroup (two at the tile's edge).
-//   bound: memory.  NCHW -> NHWC of [32, 128, 56, 56]: float32 37.5 us a call
-//   with one unit per output chunk, 15.6 here (6.6 TB/s); bfloat16 30.5 -> 9.7,
-//   float64 129 -> 29.7; a [3000, 4000] float32 matrix 67.3 -> 15.6.
+//   bound: memory.  NCHW -> NHWC of [32, 128, 56, 56], repeated on the same
+//   arrays (in the 256 MB cache): float32 37.5 us a call with one unit per
+//   output chunk, 15.6 here (6.6 TB/s); bfloat16 30.5 -> 9.7, float64 129 ->
+//   29.7; a [3000, 4000] float32 matrix 67.3 -> 15.6.  Over arrays past the
+//   cache the float32 images take 36.6 -> 20.1 (5.1 TB/s, a copy's rate).
 //   Plain accesses: non-temporal ones leave float32 as it is and cost float64
 //   30 -> 38 us (a tile's rows end inside lines that its neighbour completes).
 //   tile: 64 elements are 128 to 512 bytes either way; 17 KB of LDS (33 for
