@@ -395,7 +395,12 @@ xg_status xg_plan_scan(const xg_expr* e, const xg_scan_desc* s, const xg_tensor*
  * minmax, immediate evaluation, extents past 2^31 elements) are planned as
  * their descriptors and run as xg_reduce / xg_scan on every execution: the
  * host plans them each time, and a first execution may grow the stream's
- * workspace, so run such a plan once before capturing it in a graph. */
+ * workspace, so run such a plan once before capturing it in a graph.  (Scans
+ * of an expression that xg_scan evaluates first are planned that way too.)
+ * A reduction of a small expression without a compiled kernel evaluates the
+ * expression into its workspace and reduces it there; executed without one
+ * (workspace NULL) on a stream that is being captured, it reduces the
+ * expression in one launch instead, and its fold order may then differ. */
 /* xg_assign_reduce2d prepared: XG_UNSUPPORTED when the single pass does not
  * apply to these descriptors (then plan the assignment and the reductions
  * apart). */
@@ -405,7 +410,8 @@ xg_status xg_plan_assign_reduce2d(const xg_expr* e, const xg_tensor* out, const 
 /* Bytes of device workspace the plan needs (0 for most elementwise plans). */
 size_t xg_plan_workspace_size(xg_plan_t plan);
 /* Enqueue the plan on `stream`; `workspace` must hold xg_plan_workspace_size
- * bytes (NULL: the library's per-stream workspace is used). */
+ * bytes (NULL: the library's per-stream workspace is used, which a later,
+ * larger call on that stream frees: give captured plans a block of their own). */
 xg_status xg_plan_execute(xg_plan_t plan, void* workspace, xg_stream_t stream);
 /* Enqueue n plans that do not read each other's outputs.  Elementwise plans
  * that run the same compiled program at the same normalised rank are fused

@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <utility>
@@ -99,6 +100,23 @@ void* workspace(size_t bytes, hipStream_t stream) {
         b.bytes = n;
     }
     return b.ptr;
+}
+
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &s) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return s != hipStreamCaptureStatusNone;
+}
+
+size_t workspace_held(hipStream_t stream) {
+    int dev = 0;
+    check_hip(hipGetDevice(&dev), "hipGetDevice");
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    const auto f = g_ws.find(WsKey{dev, reinterpret_cast<void*>(stream)});
+    return f == g_ws.end() ? 0 : f->second.bytes;
 }
 
 namespace {
@@ -490,6 +508,34 @@ struct EvalFirst {
     EvalFirst(const EvalFirst&) = delete;
 };
 
+// Both launches of such a reduction, planned; they share one block (16-byte
+// aligned) of bytes() bytes: the temporary, then the reduction's partials.
+struct EvalFirstPlan {
+    EwPlan ew;
+    RedPlan red;
+    int Vw = 4, V = 4;
+    size_t tmp = 0;
+    EvalFirstPlan(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out) {
+        EvalFirst f(e);
+        f.t.data = reinterpret_cast<void*>(kSizingBase);
+        ew = plan_assign_best(e, &f.t, &Vw);
+        red = plan_reduce_best(&f.e, r, out, &V);
+        tmp = f.bytes;
+    }
+    size_t bytes() const { return tmp + reduce_workspace_bytes(red); }
+    hipError_t launch(char* block, hipStream_t st, const char** used) const {
+        EwPlan a = ew;
+        a.out_ptr = block;
+        const hipError_t err = launch_ew(a, Vw, device_cus(), st, nullptr);
+        if (err != hipSuccess) return err;
+        RedPlan q = red;
+        q.leaves[0].ptr = block;  // the program of a lone array has one leaf
+        q.partials = reduce_workspace_bytes(red) ? block + tmp : nullptr;
+        q.counters = nullptr;
+        return launch_reduce(q, V, st, used);
+    }
+};
+
 // A reduction plan_reduce handles (every op but minmax; variance / stddev of
 // the deviation expression), in pieces when its reduced extent is too long.
 void reduce_plain(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out, hipStream_t st, Arena& a,
@@ -763,15 +809,8 @@ void xg::reduce_call(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor*
             whole = false;  // in pieces, or refused, below
         }
         if (whole && counters && reduce_eval_first_ok(e, p, V)) {
-            EvalFirst f(e);
-            f.t.data = reinterpret_cast<void*>(kSizingBase);
-            p = plan_reduce_best(&f.e, r, out, &V);
-            char* block = src(f.bytes + reduce_workspace_bytes(p), st, ctx);
-            f.t.data = block;
-            p.leaves[0].ptr = block;  // the program of a lone array has one leaf
-            p.partials = reduce_workspace_bytes(p) ? block + f.bytes : nullptr;
-            assign_launch(e, &f.t, st, nullptr);
-            check_hip(launch_reduce(p, V, st, &used), "reduction launch");
+            const EvalFirstPlan f(e, r, out);
+            check_hip(f.launch(src(f.bytes(), st, ctx), st, &used), "reduction launch");
             note_kernel(used ? used : "empty");
             return;
         }
@@ -1195,6 +1234,28 @@ struct xg_plan_s {
                                       : xg_scan(&e, &d_scan, &d_out, reinterpret_cast<xg_stream_t>(st));
         if (r != XG_OK) raise(r, xg_last_error_message());
     }
+    // kind 1 of a small expression (reduce_eval_first_ok): the two launches that
+    // run in a block of `ws` bytes; `red` alone runs where there is none
+    std::unique_ptr<EvalFirstPlan> first;
+    void reduce(void* block, hipStream_t st, const char** used) {
+        if (!red.n_out) return;
+        bool merge_here = !block;  // with the stream's counters
+        if (first) {
+            // under capture the library's workspace is no place for the
+            // temporary (a larger call later frees it, and the graph keeps its
+            // address), and the counters may not be allocated yet
+            if (!block && !capturing(st)) block = workspace(ws, st);
+            if (block && reinterpret_cast<uintptr_t>(block) % 16 == 0) {
+                check_hip(first->launch(static_cast<char*>(block), st, used), "reduction launch");
+                return;
+            }
+            merge_here = false;
+        }
+        const size_t bytes = reduce_workspace_bytes(red);
+        red.partials = bytes ? (block ? block : workspace(bytes, st)) : nullptr;
+        red.counters = merge_here ? reduce_counters(st) : nullptr;
+        check_hip(launch_reduce(red, V, st, used), "reduction launch");
+    }
     xg::EwPlan ew;
     std::vector<std::pair<xg::EwPlan, int>> pieces;  // assign past 32-bit offsets: one plan per piece (ew unused)
     xg::RedPlan red;
@@ -1240,7 +1301,10 @@ xg_status xg_plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_ten
                 try {
                     p->red = plan_reduce_best(e, r, out, &p->V);
                     p->ws = reduce_workspace_bytes(p->red);
-                    deferred = reduce_eval_first_ok(e, p->red, p->V);
+                    if (reduce_eval_first_ok(e, p->red, p->V)) {
+                        p->first = std::make_unique<EvalFirstPlan>(e, r, out);
+                        p->ws = std::max(p->ws, p->first->bytes());
+                    }
                 } catch (const Error& err) {
                     if (err.code != XG_UNSUPPORTED) throw;
                     deferred = true;  // past 32-bit indexing: xg_reduce cuts it into pieces
@@ -1307,11 +1371,7 @@ xg_status xg_plan_execute(xg_plan_t p, void* ws, xg_stream_t stream) {
             if (p->ew.units) check_hip(launch_ew(p->ew, p->V, device_cus(), st, &used), "elementwise launch");
             for (const auto& pc : p->pieces) check_hip(launch_ew(pc.first, pc.second, device_cus(), st, &used), "elementwise launch");
         } else if (p->kind == 1) {
-            if (p->red.n_out) {
-                p->red.partials = p->ws ? (ws ? ws : workspace(p->ws, st)) : nullptr;
-                p->red.counters = ws ? nullptr : reduce_counters(st);
-                check_hip(launch_reduce(p->red, p->V, st, &used), "reduction launch");
-            }
+            p->reduce(ws, st, &used);
         } else if (p->kind == 3) {
             launch_assign_rc(p->arc, p->ws ? (ws ? ws : workspace(p->ws, st)) : nullptr, st);
             used = "assign_rc";
@@ -1368,10 +1428,8 @@ xg_status xg_plan_execute_many(const xg_plan_t* plans, int64_t n, xg_stream_t st
         for (int64_t i = 0; i < n; ++i) {
             xg_plan_s* p = plans[i];
             const char* used = nullptr;
-            if (p->kind == 1 && p->red.n_out) {
-                p->red.partials = p->ws ? workspace(p->ws, st) : nullptr;
-                p->red.counters = reduce_counters(st);
-                check_hip(launch_reduce(p->red, p->V, st, &used), "reduction launch");
+            if (p->kind == 1) {
+                p->reduce(nullptr, st, &used);
             } else if (p->kind == 3) {
                 launch_assign_rc(p->arc, p->ws ? workspace(p->ws, st) : nullptr, st);
             } else if (p->kind >= 4) {

@@ -18,6 +18,10 @@ void note_kernel(const char* name);
 void check_hip(hipError_t e, const char* what);
 // per (device, stream) scratch buffer of at least `bytes`
 void* workspace(size_t bytes, hipStream_t stream);
+// what the stream's scratch buffer holds now
+size_t workspace_held(hipStream_t stream);
+// the stream is being captured in a graph (or cannot say)
+bool capturing(hipStream_t stream);
 // device address of xg_reduce_noalloc's fixed per-device array, resolved
 // once per device (the current one)
 char* scratch_setup();

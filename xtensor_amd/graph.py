@@ -9,13 +9,15 @@ of the plans themselves.
 The plans keep their operands alive and read whatever those hold at replay
 time, as `Plan.run()` does.  Before capturing, every plan runs once on the
 graph's own stream, so one-time work (run-time compiles, workspace growth)
-stays out of the graph.  The captured launches use that stream's workspace:
-replays of one `PlanGraph` must not overlap (successive replays on one stream
-are fine).
+stays out of the graph.  The captured launches share one workspace, which the
+`PlanGraph` owns (plans kept as descriptors, a variance or a scan of an
+expression for example, use the stream's): replays of one `PlanGraph` must not
+overlap (successive replays on one stream are fine).
 """
 
 from __future__ import annotations
 
+import ctypes as C
 from typing import Sequence
 
 from .core import Plan
@@ -35,12 +37,21 @@ class PlanGraph:
         for p in self.plans:
             p.run(stream=handle)
         self._stream.synchronize()
+        # the plans' workspace: the stream's own is freed when a later, larger
+        # call on that stream grows it
+        need = max(p._workspace_size() for p in self.plans)
+        self._block = torch.empty(need, dtype=torch.uint8, device="cuda") if need else None
+        block = self._block.data_ptr() if need else None
         self._graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self._graph, stream=self._stream):
             for p in self.plans:
-                p.run(stream=handle)
+                p._run_in(block, C.c_void_p(handle))
         torch.cuda.current_stream().wait_stream(self._stream)
 
     def replay(self) -> None:
         """Enqueue every captured launch, in order, on the current stream."""
+        if self._block is not None:
+            import torch
+
+            self._block.record_stream(torch.cuda.current_stream())
         self._graph.replay()
