@@ -294,7 +294,10 @@ xg_status xg_reduce_info(const xg_expr* e, const xg_reduce_desc* r, int32_t* dty
  * out must have exactly the reduction's shape; its dtype may differ from the
  * result dtype (then values are static_cast on store).  sum / prod / amax /
  * amin accept a reduced dimension past 2^31 elements: it is reduced in
- * pieces through a temporary of the result's size per piece. */
+ * pieces through a temporary of the result's size per piece.  A small
+ * expression without a compiled kernel is evaluated into the stream's
+ * workspace and reduced there; on a stream that is being captured it is
+ * reduced in one launch instead, whose fold order may differ. */
 xg_status xg_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out, xg_stream_t stream);
 
 /* out = reduce(e, axes) exactly as xg_reduce, for callers that cannot

@@ -105,3 +105,50 @@ def test_plan_graph_and_many():
         with torch.cuda.stream(g._stream):
             xt.cumsum(xt.zeros(((1 << 21) + (1 << 20) * rep,), "float32") + 1.0)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("shape,dtype,axes", CASES)
+def test_eager_call_captured(shape, dtype, axes):
+    """A captured xg_reduce that is not split keeps no address of the stream's
+    workspace: its replays are right after the workspace has grown.  (A split
+    one keeps its partials there, so it is replayed without growing it.)"""
+    import torch
+    r, out, want, mag = _make(shape, dtype, axes)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        xt.noalias(out).assign(r)  # one eager pass
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        xt.noalias(out).assign(r)
+    for rep in range(3):
+        xt.noalias(out).assign(out * 0)
+        g.replay()
+        torch.cuda.synchronize()
+        _check(out, want, mag, dtype)
+        if shape == (1029, 575) and axes == [1]:  # 1029 outputs: no split
+            with torch.cuda.stream(s):
+                xt.cumsum(xt.zeros(((1 << 20) * (rep + 1),), "float32") + 1.0)
+            torch.cuda.synchronize()
+
+
+def test_captured_variance_matches_eager():
+    """Its mean is in the stream's workspace anyway; captured after an eager
+    pass it runs the same kernels."""
+    import torch
+    rng = np.random.default_rng(3)
+    a = xt.from_numpy(rng.normal(size=(200, 300)).astype("float32"))
+    r = xt.variance(a * a + a, [1])
+    out = xt.empty(r.shape, r.dtype)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        want = xt.eval(r).to_numpy()
+        g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        xt.noalias(out).assign(r)
+    for _ in range(3):
+        xt.noalias(out).assign(out * 0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert out.to_numpy().tobytes() == want.tobytes()

@@ -791,8 +791,12 @@ void reduce_top(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out,
 }  // namespace
 
 void xg::reduce_call(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out, hipStream_t st, BlockSource src,
-                     void* ctx, bool counters) {
+                     void* ctx, bool counters, size_t first_room) {
     const char* used = nullptr;
+    // a stream's own block, under capture: it may not grow, and a graph that
+    // needs no block otherwise is not to keep the address of one that a larger
+    // call later frees
+    auto held = [&] { return counters && capturing(st); };
     // one plan and at most one block (its split partials): planned once
     const bool lone = e && r && !(r->flags & ~XG_REDUCE_IMMEDIATE) &&
                       (!(r->flags & XG_REDUCE_IMMEDIATE) ||
@@ -808,15 +812,21 @@ void xg::reduce_call(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor*
             if (err.code != XG_UNSUPPORTED) throw;
             whole = false;  // in pieces, or refused, below
         }
-        if (whole && counters && reduce_eval_first_ok(e, p, V)) {
-            const EvalFirstPlan f(e, r, out);
-            check_hip(f.launch(src(f.bytes(), st, ctx), st, &used), "reduction launch");
-            note_kernel(used ? used : "empty");
-            return;
-        }
         if (whole) {
             if (p.n_out) {
                 const size_t bytes = reduce_workspace_bytes(p);
+                if (first_room && reduce_eval_first_ok(e, p, V)) {
+                    if (!held()) {
+                        const EvalFirstPlan f(e, r, out);
+                        const size_t n = std::max(bytes, f.bytes());  // enough for the same call captured later
+                        if (n <= first_room) {
+                            check_hip(f.launch(src(n, st, ctx), st, &used), "reduction launch");
+                            note_kernel(used ? used : "empty");
+                            return;
+                        }
+                    }
+                    counters = false;
+                }
                 p.partials = bytes ? src(bytes, st, ctx) : nullptr;
                 p.counters = counters ? reduce_counters(st) : nullptr;
                 check_hip(launch_reduce(p, V, st, &used), "reduction launch");
@@ -826,10 +836,15 @@ void xg::reduce_call(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor*
         }
     }
     Arena sizing;
-    sizing.eval_first = counters;  // callers with a fixed block keep its size to the partials
+    if (held()) first_room = workspace_held(st);
+    sizing.eval_first = first_room > 0;
     reduce_top(e, r, out, st, sizing, &used);
+    if (sizing.eval_first && sizing.used > first_room) {
+        sizing = Arena{};
+        reduce_top(e, r, out, st, sizing, &used);
+    }
     Arena a;
-    a.eval_first = counters;
+    a.eval_first = sizing.eval_first;
     a.measure = false;
     a.cap = sizing.used;
     a.base = sizing.used ? src(sizing.used, st, ctx) : nullptr;
@@ -887,7 +902,7 @@ xg_status xg_reduce_info(const xg_expr* e, const xg_reduce_desc* r, int32_t* dty
 }
 
 xg_status xg_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out, xg_stream_t stream) {
-    return guard([&] { reduce_call(e, r, out, reinterpret_cast<hipStream_t>(stream), stream_workspace, nullptr, true); });
+    return guard([&] { reduce_call(e, r, out, reinterpret_cast<hipStream_t>(stream), stream_workspace, nullptr, true, SIZE_MAX); });
 }
 
 xg_status xg_assign_reduce2d(const xg_expr* e, const xg_tensor* out, const xg_reduce_desc* row_red,
@@ -916,8 +931,8 @@ xg_status xg_assign_reduce2d(const xg_expr* e, const xg_tensor* out, const xg_re
         le.n_leaves = 1;
         le.nodes = &leaf;
         le.leaves = &ol;
-        if (row_red) reduce_call(&le, row_red, row_out, st, stream_workspace, nullptr, true);
-        if (col_red) reduce_call(&le, col_red, col_out, st, stream_workspace, nullptr, true);
+        if (row_red) reduce_call(&le, row_red, row_out, st, stream_workspace, nullptr, true, SIZE_MAX);
+        if (col_red) reduce_call(&le, col_red, col_out, st, stream_workspace, nullptr, true, SIZE_MAX);
         note_kernel("assign_then_reduce");
     });
 }

@@ -322,7 +322,7 @@ struct xg_server_s {
         if (r0.tpl == XG_TPL_REDUCE) {
             for (const Job& j : s.jobs) {
                 const xg_expr e = j.expr();
-                reduce_call(&e, &j.rd, &j.out, s.stream, slot_workspace, nullptr, true);
+                reduce_call(&e, &j.rd, &j.out, s.stream, slot_workspace, nullptr, true, SIZE_MAX);
             }
             std::lock_guard<std::mutex> lk(mu);
             ++launches;

@@ -52,9 +52,12 @@ using BlockSource = char* (*)(size_t bytes, hipStream_t stream, void* ctx);
 // out = reduce(e) (every reduction kind of xg_reduce), with its temporaries
 // and split partials in one block from `src`; `counters`: the column
 // reductions may merge their splits themselves with the stream's arrival
-// counters (allocated on first use), else a combine kernel does.
+// counters (allocated on first use), else a combine kernel does.  A small
+// expression without a compiled kernel is evaluated into the block first as
+// long as the block stays within `first_room` bytes (0: never), and reduced in
+// one launch otherwise.
 void reduce_call(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out, hipStream_t stream,
-                 BlockSource src, void* ctx, bool counters);
+                 BlockSource src, void* ctx, bool counters, size_t first_room);
 
 // the stream's arrival counters (zeroed, kReduceCounters words)
 uint32_t* reduce_counters(hipStream_t stream);
