@@ -303,14 +303,16 @@ xg_status xg_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
 /* out = reduce(e, axes) exactly as xg_reduce, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in xtensor.  The call's
- * temporaries (split partials, a variance's kept-dims mean, an immediate
- * reduction's evaluated expression, the pieces of a reduction past 32-bit
- * indexing) live in one fixed array per device of
+ * temporaries (split partials, a variance's kept-dims mean, the evaluated
+ * expression of an immediate reduction or of a small one without a compiled
+ * kernel, the pieces of a reduction past 32-bit indexing) live in one fixed array per device of
  * xg_reduce_noalloc_max_bytes() bytes (16 MiB), held until the process ends;
  * a reduction that needs more returns XG_OUT_OF_MEMORY before enqueueing
  * anything.  It calls no hipMalloc / hipFree and loads no module: a run-time
  * compiled kernel is used only if this process has already loaded it (else
- * the ahead-of-time or generic kernels run).  Every call on one device
+ * the ahead-of-time or generic kernels run), and a small expression whose
+ * values do not fit the array beside the other temporaries is reduced in one
+ * launch: in these two cases the fold order may differ.  Every call on one device
  * shares that array: calls that overlap in time on one device (two streams,
  * or two threads) race and must be serialised by the caller. */
 xg_status xg_reduce_noalloc(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* out, xg_stream_t stream);

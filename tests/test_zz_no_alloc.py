@@ -94,6 +94,39 @@ def test_noalloc_matches_xg_reduce_twice(idx):
             assert _rel(got, want) <= tol, f"{name}: rel err {_rel(got, want)}"
 
 
+@pytest.mark.parametrize("shape", [(1029, 575), (300, 41), (7, 5), (3, 20001), (60000, 3)])
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+def test_noalloc_small_expressions(shape, dtype):
+    """Expressions without a compiled kernel: both calls evaluate first and
+    merge in the same order (uncompensated products included, whose last bits
+    depend on it)."""
+    rng = np.random.default_rng(sum(shape))
+    h = rng.uniform(0.9, 1.1, shape).astype(dtype)
+    a = xt.from_numpy(h)
+    v = (h * h + np.asarray(0.5, dtype) * h).astype(np.float64)
+    e = a * a + xt.scalar(0.5, dtype) * a
+    for axes in ([0], [1], None):
+        ax = None if axes is None else tuple(axes)
+        for r, want in ((xt.sum(e, axes), v.sum(ax)), (xt.prod(xt.sqrt(e) / 1.2, axes), None), (xt.amax(e, axes), v.max(ax)),
+                        (xt.norm_l2(e, axes), np.sqrt((v * v).sum(ax))), (xt.variance(e, axes), v.var(ax))):
+            ref, got = _both(r)
+            assert got.tobytes() == ref.tobytes(), f"{r.kind} {axes} of {dtype} {shape}"
+            if want is not None:
+                assert _rel(got, want) <= 1e-5, (r.kind, axes)
+
+
+def test_noalloc_small_expression_beyond_its_scratch():
+    """A variance over an axis of one element: its mean, the values and the
+    deviations, 8 MiB each, do not fit the array; in one launch they do."""
+    n = (1 << 20) - 1
+    a = xt.from_numpy(np.arange(n, dtype=np.float64).reshape(n, 1))
+    r = xt.variance(a * 2.0 + a, [1])
+    out = xt.from_numpy(np.full(n, 5.0))
+    assert _call(A.lib().xg_reduce_noalloc, r, out) == A.OK, A.lib().xg_last_error_message()
+    _sync()
+    assert not out.to_numpy().any()
+
+
 def test_noalloc_allocates_nothing():
     import torch
     rng = np.random.default_rng(5)

@@ -2,15 +2,17 @@
 // allocate device memory (code under HIP graph capture, tight serving loops).
 //
 // A reduction's temporaries (split partials, the kept-dims mean of a
-// variance, the evaluated expression of an immediate reduction, the pieces
-// of a reduction past 32-bit indexing) come from `scratch`, one fixed array
+// variance, the evaluated expression of an immediate reduction or of a small
+// one without a compiled kernel, the pieces of a reduction past 32-bit
+// indexing) come from `scratch`, one fixed array
 // per device that lives as long as the process, instead of the library's
 // per-stream workspace.  The call plans twice as xg_reduce does (a sizing
 // pass, then the real one) and rejects a reduction whose temporaries exceed
 // the array.  Kernels are the ones xg_reduce launches, except that a
 // run-time compiled kernel is used only when this process has already loaded
-// it (no compile, no module load); otherwise the ahead-of-time or generic
-// kernels run.
+// it (no compile, no module load; otherwise the ahead-of-time or generic
+// kernels run), and that a small expression whose evaluated values would not
+// fit the array beside the other temporaries is reduced in one launch.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -71,7 +73,7 @@ xg_status xg_reduce_noalloc(const xg_expr* e, const xg_reduce_desc* r, const xg_
         scratch_setup();
         const int prev = jit_set_thread_loaded_only(1);
         try {
-            reduce_call(e, r, out, reinterpret_cast<hipStream_t>(stream), scratch_block, nullptr, false, 0);
+            reduce_call(e, r, out, reinterpret_cast<hipStream_t>(stream), scratch_block, nullptr, false, kScratchBytes);
         } catch (...) {
             jit_set_thread_loaded_only(prev);
             throw;
