@@ -99,6 +99,48 @@ template <class T> __device__ __forceinline__ T sub_max(T m, int lpr) {
     return m;
 }
 
+// The same for RB independent values with a run-time `lpr`: a level's RB
+// exchanges go out together.  One value after the other, each with a loop of
+// its own, left a wave waiting for RB * log2(lpr) exchanges in turn: the
+// 4096-instance softmax with tasks of 4096 elements took 217 us a replay that
+// way and 194 this way, 320 and 212 with tasks of 8192 (with one code form per
+// lane count: 199 and 219).
+// (Float64 pairs four at a time: eight and their partners do not fit the
+// registers of five waves a SIMD.)
+template <int RB, class A> __device__ __forceinline__ void sub_combine_rows(A (&a)[RB], int lpr) {
+    constexpr int N = sizeof(A) > 8 && RB > 4 ? 4 : RB;
+    static_assert(RB % N == 0, "whole parts");
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int h = 0; h < RB; h += N) {
+        for (int m = 1; m < lpr; m <<= 1) {
+            A o[N];
+#pragma unroll
+            for (int g = 0; g < N; ++g) o[g] = a[h + g].shfl_xor(m);
+#pragma unroll
+            for (int g = 0; g < N; ++g) {
+                if (lane & m) {
+                    o[g].merge(a[h + g]);
+                    a[h + g] = o[g];
+                } else {
+                    a[h + g].merge(o[g]);
+                }
+            }
+        }
+    }
+}
+
+template <int RB, class T> __device__ __forceinline__ void sub_max_rows(T (&m)[RB], int lpr) {
+    const int lane = threadIdx.x & 63;
+    for (int k = 1; k < lpr; k <<= 1) {
+        T o[RB];
+#pragma unroll
+        for (int g = 0; g < RB; ++g) o[g] = __shfl_xor(m[g], k);
+#pragma unroll
+        for (int g = 0; g < RB; ++g) m[g] = (lane & k) ? fmax_x(o[g], m[g]) : fmax_x(m[g], o[g]);
+    }
+}
+
 // exp(x - m) for x <= m (m is the row maximum), without the rounding error
 // of forming x - m in the input precision: d + e == x - m exactly (TwoSum).
 //   float:  2^p with p = (d + e) * log2(e) carried as ph + pl (Dekker
@@ -171,7 +213,7 @@ constexpr uint32_t kOffNone = 0x80000000u;  // an offset past every resource
 // wave-uniform `lpr_rt`.  One form for them keeps the kernel's instructions at
 // 60 KB: with one per lane count they were 92 KB, more than the 64 KB cache two
 // CUs share, and a batch waited for its code (8 instances, one trip each: 55.9
-// us a launch, 14.7 now; 1024 instances 99.1 -> 47.6 with the schedule below).
+// us a launch, 14.7 now; 1024 instances 99.1 -> 45 with the schedule below).
 template <class T, int OP, int LPR, int NE, int RB>
 __device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, int rb, int sub, int sl, int lpr_rt) {
     using Tr = BTraits<T>;
@@ -212,8 +254,12 @@ __device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, 
 #pragma unroll
             for (int k = 1; k < NE; ++k) m[g] = OP == BO_SOFTMAX ? max_num(m[g], v[g][k]) : fmax_x(m[g], v[g][k]);
         }
+        if constexpr (LPR == 0) {
+            sub_max_rows(m, lpr);
+        } else {
 #pragma unroll
-        for (int g = 0; g < RB; ++g) m[g] = sub_max(m[g], lpr);
+            for (int g = 0; g < RB; ++g) m[g] = sub_max(m[g], LPR);
+        }
     }
     if constexpr (OP == BO_MAX) {
 #pragma unroll
@@ -235,8 +281,12 @@ __device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, 
                 s[g].add(Tr::reg(v[g][k]));
             }
         }
+        if constexpr (LPR == 0) {
+            sub_combine_rows(s, lpr);
+        } else {
 #pragma unroll
-        for (int g = 0; g < RB; ++g) s[g] = sub_combine(s[g], lpr);
+            for (int g = 0; g < RB; ++g) s[g] = sub_combine(s[g], LPR);
+        }
 #pragma unroll
         for (int g = 0; g < RB; ++g) {
             const int r = rb + g * PER + sub;
