@@ -590,6 +590,7 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
         // enough loads in flight to cover HBM latency
         const uint64_t target_waves = uint64_t(cus) * uint64_t(g_reduce_waves_per_cu);
         constexpr uint64_t kU = 4;                          // chunks (rows) in flight per lane
+        bool latency_bound = false;                         // rows: too short for that
         if (p.layout == RL_ROWS) {
             const uint64_t chunks = p.red_count;
             uint64_t g = pow2_ceil(uint32_t(std::max<uint64_t>(1, (chunks + 2 * kU - 1) / (2 * kU))));
@@ -598,8 +599,14 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
             const uint64_t waves = (uint64_t(n_out) * p.f_group + 63) / 64;
             uint64_t s = 1;
             if (waves < target_waves) {
-                s = (target_waves + waves - 1) / waves;
-                s = std::min<uint64_t>(s, std::max<uint64_t>(1, chunks / (uint64_t(p.f_group) * kU * 2)));
+                // rounded down: a few waves past the target run beside or after
+                // the even ones (row sums, rounded up -> this: float32 [9, 1604244]
+                // 17.8 -> 15.3 us, [2739, 9187] 23.0 -> 19.3, [300, 500000] 110.7
+                // -> 97.0, bfloat16 [2773, 9075] 16.8 -> 12.7)
+                s = target_waves / waves;
+                const uint64_t most = std::max<uint64_t>(1, chunks / (uint64_t(p.f_group) * kU * 2));
+                latency_bound = most < s;
+                s = std::min(s, most);
             }
             p.f_splits = int(std::min<uint64_t>(s, 65535));
             p.f_per_split = uint32_t((chunks + p.f_splits - 1) / p.f_splits);
@@ -630,9 +637,13 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
         }
         while (p.f_splits > 1 && uint64_t(n_out) * uint64_t(p.f_splits) >= (uint64_t(1) << 31)) p.f_splits /= 2;
         p.f_per_split = uint32_t((uint64_t(p.red_count) + p.f_splits - 1) / p.f_splits);
-        if (p.layout == RL_ROWS && p.f_splits > 1) {
-            // whole rounds of kU chunks a lane: a split of 12.25 chunks a lane
-            // costs four rounds, the last one mostly dropped values
+        if (p.layout == RL_ROWS && p.f_splits > 1 && latency_bound) {
+            // Fewer waves than the GPU holds: a split's rounds of kU chunks a lane
+            // are latencies, and a split of 2.05 rounds takes three.  Whole rounds
+            // instead (the channel means of float32 [100, 33, 31, 29] 10.9 -> 10.3
+            // us, their variance 23.8 -> 22).  Where the waves fill the GPU this
+            // only changes their number, away from the even one (all of float32
+            // [9000, 7500] 50 us as it is, 60 rounded).
             const uint64_t round = uint64_t(p.f_group) * kU;
             const uint64_t k = std::max<uint64_t>(1, (p.f_per_split + round / 2) / round);
             const uint64_t s = (uint64_t(p.red_count) + k * round - 1) / (k * round);
