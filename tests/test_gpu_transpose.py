@@ -1,10 +1,13 @@
 """Copies between layouts contiguous along different dimensions, by tiles of
 64 x 64 through LDS: the copy itself against numpy, bit for bit."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import xtensor_amd as xt
+from xtensor_amd import _abi as A
 
 pytestmark = pytest.mark.gpu
 
@@ -17,23 +20,28 @@ def distinct(shape, dtype):
     return (np.arange(n, dtype=np.int64) * 7919 % 30011).astype(dtype).reshape(shape)
 
 
-def copied(view, dtype, fill=None):
-    out = xt.zeros(view.shape, str(np.dtype(dtype))) if fill is None else fill
+def copied(view, dtype, tiles=True):
+    """The copy; tiles: whether the tiles' kernel makes it (None: either)."""
+    out = xt.zeros(view.shape, str(np.dtype(dtype)))
     xt.noalias(out).assign(view)
+    if tiles is not None:
+        assert (xt.last_kernel() == "transpose") == tiles
     return out.to_numpy()
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("c,hw", EDGES)
 def test_matrix_and_images(c, hw, dtype):
-    """Edges of a tile either way, with none, one and two other dimensions."""
+    """Edges of a tile either way, with none, one and two other dimensions; a
+    tile of 17 x 64 is just below the line."""
+    tiles = (c, hw) != (17, 64)
     x = distinct((c, hw), dtype)
-    assert np.array_equal(copied(xt.transpose(xt.from_numpy(x), (1, 0)), dtype), x.T)
+    assert np.array_equal(copied(xt.transpose(xt.from_numpy(x), (1, 0)), dtype, tiles), x.T)
     x = distinct((3, c, hw), dtype)
-    assert np.array_equal(copied(xt.transpose(xt.from_numpy(x), (0, 2, 1)), dtype), x.transpose(0, 2, 1))
+    assert np.array_equal(copied(xt.transpose(xt.from_numpy(x), (0, 2, 1)), dtype, tiles), x.transpose(0, 2, 1))
     x = distinct((2, c, 3, hw), dtype)
     assert np.array_equal(copied(xt.transpose(xt.from_numpy(x), (2, 3, 0, 1)), dtype), x.transpose(2, 3, 0, 1))
-    assert np.array_equal(copied(xt.transpose(xt.from_numpy(x), (0, 3, 2, 1)), dtype), x.transpose(0, 3, 2, 1))
+    assert np.array_equal(copied(xt.transpose(xt.from_numpy(x), (0, 3, 2, 1)), dtype, tiles), x.transpose(0, 3, 2, 1))
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -44,6 +52,7 @@ def test_parts_of_arrays(dtype):
     part = xt.view(xt.from_numpy(x), xt.range_(1, 68), xt.range_(3, 200))
     whole = xt.from_numpy(np.full((230, 90), 7, dtype))
     xt.noalias(xt.view(whole, xt.range_(5, 202), xt.range_(1, 68))).assign(xt.transpose(part, (1, 0)))
+    assert xt.last_kernel() == "transpose"
     want = np.full((230, 90), 7, dtype)
     want[5:202, 1:68] = x[1:68, 3:200].T
     assert np.array_equal(whole.to_numpy(), want)
@@ -56,9 +65,11 @@ def test_bfloat16_bits():
     x, by_tiles, by_elements = (xt.zeros(s, "bfloat16") for s in ((128, 512), (512, 128), (512, 128)))
     x.storage.view(torch.int16)[:65536].copy_(torch.from_numpy(bits.view(np.int16).ravel()))
     xt.noalias(by_tiles).assign(xt.transpose(x, (1, 0)))
+    assert xt.last_kernel() == "transpose"
     for r in range(0, 128, 16):   # 16 columns at a time are below the tiles' line
         part = xt.transpose(xt.view(x, xt.range_(r, r + 16), xt.all_()), (1, 0))
         xt.noalias(xt.view(by_elements, xt.all_(), xt.range_(r, r + 16))).assign(part)
+        assert xt.last_kernel() != "transpose"
     got, ref = (o.storage.view(torch.int16)[:65536].cpu().numpy() for o in (by_tiles, by_elements))
     assert np.array_equal(got, ref)
     nan = (bits & 0x7FFF) > 0x7F80
@@ -80,3 +91,20 @@ def test_prepared_and_graph_replays():
         torch.cuda.synchronize()
         want = (x + np.float32(k + 1)).transpose(0, 2, 3, 1)
         assert np.array_equal(direct.to_numpy(), want) and np.array_equal(replayed.to_numpy(), want)
+
+
+@pytest.mark.parametrize("dtype", ["int16", "float32", "float64"])
+def test_large_copy_compiles_nothing(dtype):
+    """Past the run-time compiler's threshold too: no kernel is compiled,
+    loaded or looked up for a copy that goes by tiles."""
+    x = distinct((1100, 1000), np.dtype(dtype))
+    d = xt.from_numpy(x)
+    before, after = ((C.c_int64 * 4)() for _ in range(2))
+    L = A.lib()
+    L.xg_debug_jit_stats(before)
+    got = copied(xt.transpose(d, (1, 0)), np.dtype(dtype))
+    plan_out = xt.zeros((1000, 1100), dtype)
+    xt.plan(plan_out, xt.transpose(d, (1, 0))).run()
+    L.xg_debug_jit_stats(after)
+    assert list(before) == list(after)
+    assert np.array_equal(got, x.T) and np.array_equal(plan_out.to_numpy(), x.T)

@@ -158,12 +158,13 @@ char* Arena::take(size_t bytes) {
 
 using namespace xg;
 
-// plan with the compiled-kernel vector width; without a matching compiled
-// program, re-plan for the generic interpreter
+// plan with the compiled-kernel vector width (a transposed copy by tiles, at
+// any width, compiles nothing); without a matching compiled program, re-plan
+// for the generic interpreter
 EwPlan xg::plan_assign_best(const xg_expr* e, const xg_tensor* out, int* V) {
     *V = choose_vector_width(e, out);
     EwPlan p = plan_assign(e, out, *V);
-    if (!ew_find_spec(p, *V) && !ew_jit_ok(p, *V)) {
+    if (!ew_find_spec(p, *V) && !ew_takes_tiles(p) && !ew_jit_ok(p, *V)) {
         const int w = ew_interp_width(p);
         if (*V != w) p = plan_assign(e, out, *V = w);
     }

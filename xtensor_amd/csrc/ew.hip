@@ -90,6 +90,8 @@ int ew_set_thread_force_dynamic(int on) {
     return prev;
 }
 
+bool ew_takes_tiles(const EwPlan& p) { return !force_dynamic() && ew_is_transpose(p); }
+
 bool ew_jit_ok(const EwPlan& p, int V) {
     return !force_dynamic() && p.compact && jit_wanted(p.units * uint64_t(V)) && jit_ew(p, V) != nullptr;
 }
@@ -157,7 +159,7 @@ hipError_t launch_ew_multi(int spec_index, int rank, const CompactPlan* d_plans,
 hipError_t launch_ew(const EwPlan& p, int V, int cus, hipStream_t stream, const char** used) {
     if (p.units == 0) return hipSuccess;
     dim3 grid(ew_grid(p.units, cus)), block(256);
-    if (!force_dynamic() && ew_is_transpose(p)) {
+    if (ew_takes_tiles(p)) {
         if (used) *used = "transpose";
         return launch_ew_transpose(p, stream);
     }
