@@ -65,3 +65,20 @@ def test_refusals():
     host = xt.empty((4,), "float32", device="cpu")
     with pytest.raises(RuntimeError, match="device"):
         core._pack(host + a, None).assign(host, 0)
+
+
+def test_nodes_are_ordinary_objects():
+    """Expression nodes take weak references, attributes, copies and every
+    pickle protocol, as any instance does."""
+    import copy
+    import pickle
+    import weakref
+    a = core._Placeholder(A.FLOAT32, (4,))
+    s = xt.scalar(3, "int64")
+    for e in (a + s, -(a * a), s):
+        assert weakref.ref(e)() is e
+        e.note = "kept"
+        assert vars(e)["note"] == "kept" and copy.copy(e).note == "kept"
+    for protocol in range(pickle.HIGHEST_PROTOCOL + 1):
+        e = pickle.loads(pickle.dumps(s + 2, protocol))
+        assert raw(e) == raw(s + 2)

@@ -126,8 +126,6 @@ def _operator(name):
 class Expr:
     """A node of a lazy expression tree (xfunction / xscalar / container)."""
 
-    __slots__ = ()
-
     # ---- arithmetic operators (core/xoperation.hpp:231-545)
     __add__, __radd__ = _operator("PLUS")
     __sub__, __rsub__ = _operator("MINUS")
@@ -179,8 +177,6 @@ class Expr:
 class Scalar(Expr):
     """xt::xscalar leaf: a value with a C++ type (containers/xscalar.hpp)."""
 
-    __slots__ = ("dtype_code", "value")
-
     def __init__(self, value, dtype=None):
         if dtype is None:
             if isinstance(value, (bool, np.bool_)):
@@ -221,8 +217,6 @@ def _wrap(x) -> Expr:
 
 class Func(Expr):
     """xfunction node: functor `op` applied to argument expressions."""
-
-    __slots__ = ("op", "args", "index")
 
     def __init__(self, op: int, *args, index: int = 0):
         self.op = op
