@@ -82,3 +82,12 @@ def test_nodes_are_ordinary_objects():
     for protocol in range(pickle.HIGHEST_PROTOCOL + 1):
         e = pickle.loads(pickle.dumps(s + 2, protocol))
         assert raw(e) == raw(s + 2)
+
+
+def test_host_arrays_are_refused_as_such():
+    """With and without a GPU: before torch is asked for a stream."""
+    a, s = (xt.empty(n, "float32", device="cpu") for n in ((4,), ()))
+    for call in (lambda: xt.noalias(a).assign(a + a), lambda: xt.noalias(s).assign(xt.sum(a)),
+                 lambda: xt.noalias(a).assign(a * 2)):
+        with pytest.raises(RuntimeError, match="needs device"):
+            call()

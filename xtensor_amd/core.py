@@ -815,14 +815,14 @@ def _eval_reducer(r: Reducer) -> DeviceArray:
     p = _pack(r.expr, _eval_reducer)
     dt, shp = _info(p.reduce_info(r))
     out = _empty(shp, dt)
-    st = p.reduce(r, out, _raw_stream())
+    st = p.reduce(r, out, _raw_stream)
     if st:
         _check(st)
     return out
 
 
 def _reduce_into(r: Reducer, out: DeviceArray) -> None:
-    st = _pack(r.expr, _eval_reducer).reduce(r, out, _raw_stream())
+    st = _pack(r.expr, _eval_reducer).reduce(r, out, _raw_stream)
     if st:
         _check(st)
 
@@ -835,7 +835,7 @@ def assign(out, e):
     if isinstance(e, Reducer):
         _reduce_into(e, out)
         return out
-    st = _pack(e, _eval_reducer).assign(out, _raw_stream())
+    st = _pack(e, _eval_reducer).assign(out, _raw_stream)
     if st:
         _check(st)
     return out
@@ -932,7 +932,7 @@ def eval(e) -> DeviceArray:  # noqa: A001
     p = _pack(e, _eval_reducer)
     dt, shp = _info(p.info())
     out = _empty(shp, dt)
-    st = p.assign(out, _raw_stream())
+    st = p.assign(out, _raw_stream)
     if st:
         _check(st)
     return out
@@ -1178,7 +1178,7 @@ def _scan(kind, e, axis=None, dtype=None) -> DeviceArray:
     p = _pack(e, _eval_reducer)
     dt, shp = _info(p.scan_info(op, acc, ax))
     out = _empty(shp, dt)
-    st = p.scan(op, acc, ax, out, _raw_stream())
+    st = p.scan(op, acc, ax, out, _raw_stream)
     if st:
         _check(st)
     return out

@@ -417,11 +417,15 @@ PyObject* m_scan_info(PyObject* self, PyObject* const* a, Py_ssize_t n) {
     return info_result(st, dt, nd, shape);
 }
 
-// the output's descriptor and the stream of an evaluation
+// the output's descriptor and the stream of an evaluation: its address, or a
+// function to ask for it (only once all arrays are known to be on the GPU:
+// without one torch has no stream to give)
 bool target(Packed* p, PyObject* out, PyObject* stream, xg_tensor* t, xg_stream_t* st) {
     bool cuda = p->cuda;
     if (!tensor_of(out, t, &cuda) || !on_gpu(cuda)) return false;
-    *st = reinterpret_cast<xg_stream_t>(PyLong_AsVoidPtr(stream));
+    Ref asked(PyLong_Check(stream) ? nullptr : PyObject_CallNoArgs(stream));
+    if (!asked && !PyLong_Check(stream)) return false;
+    *st = reinterpret_cast<xg_stream_t>(PyLong_AsVoidPtr(asked ? asked.p : stream));
     return !PyErr_Occurred();
 }
 
