@@ -152,3 +152,23 @@ def test_captured_variance_matches_eager():
         g.replay()
         torch.cuda.synchronize()
         assert out.to_numpy().tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("n,first", [((1 << 21) - 3, True), ((1 << 21) + 1, False)])
+def test_bound_without_the_compiler(n, first):
+    """With the run-time compiler off the temporary's 8 MiB are the bound, not
+    the compiler's threshold of 2^20 elements."""
+    L = A.lib()
+    L.xg_debug_jit(0)
+    try:
+        h = np.random.default_rng(4).normal(size=n).astype("float32")
+        a = xt.from_numpy(h)
+        r = xt.sum(a * a * 3 - a)
+        out = xt.empty(r.shape, r.dtype)
+        p = xt.plan(out, r)
+        assert (L.xg_plan_workspace_size(p.handle) >= 4 * n) == first
+        p.run()
+        v = h * h * np.float32(3) - h
+        _check(out, v.astype(np.longdouble).sum(), np.abs(v).astype(np.longdouble).sum(), "float32")
+    finally:
+        L.xg_debug_jit(1)

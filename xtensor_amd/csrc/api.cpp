@@ -469,19 +469,23 @@ bool reduce_in_pieces(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor
     return true;
 }
 
-// A reduction of an expression without a compiled kernel, below the run-time
-// compiler's threshold (p: its plan, V: the width it was made with): the
+// A reduction of an expression without a compiled kernel (p: its plan, V: the
+// width it was made with) whose values take at most kFirstBytes: the
 // expression is evaluated into a row-major temporary of its value type first,
 // as evaluation_strategy::immediate would (the same element values), and the
 // temporary reduced by the kernels a lone array has.  The generic reduction
 // kernels interpret the program with its registers in scratch memory: float32
 // sum(a * b + exp(-a * a), {1}) and amax(..., {0}) of [1029, 575] took 646 us a
-// pair that way, about 40 us this way.
+// pair that way, about 40 us this way.  By default larger expressions have a
+// kernel compiled at run time; the bound is on the temporary only (with the
+// compiler off, larger ones keep the one launch).
+constexpr int64_t kFirstBytes = int64_t(8) << 20;
 bool reduce_eval_first_ok(const xg_expr* e, const RedPlan& p, int V) {
     if (p.n_out == 0 || p.index64 || p.prog.nops < 2 || (e->n_nodes == 1 && e->nodes[0].op == XG_OP_LEAF)) return false;
     int64_t n = 1;
     for (int k = 0; k < p.rank; ++k) n *= p.shape[k];
-    return n > 0 && n < (int64_t(1) << 20) && !find_rspec(p, V) && !reduce_jit_ok(p, V);
+    if (n <= 0 || n > kFirstBytes || find_rspec(p, V) || reduce_jit_ok(p, V)) return false;
+    return n * 8 <= kFirstBytes || n * dtype_size(analyse(e).dtype) <= kFirstBytes;
 }
 
 struct EvalFirst {
