@@ -1233,13 +1233,16 @@ class Plan:
         self._exec = L.xg_plan_execute
 
     def run(self, stream=None):
-        self._run_in(None, _stream() if stream is None else C.c_void_p(stream))
+        st = _stream() if stream is None else C.c_void_p(stream)
+        r = self._exec(self.handle, None, st)
+        if r:
+            _check(r)
 
     def _workspace_size(self) -> int:
         return A.lib().xg_plan_workspace_size(self.handle)
 
     def _run_in(self, block, st) -> None:
-        """run() in a block of _workspace_size() bytes (None: the library's)."""
+        """run() in a block of _workspace_size() bytes instead of the library's."""
         r = self._exec(self.handle, block, st)
         if r:
             _check(r)
