@@ -429,8 +429,9 @@ void xg_plan_destroy(xg_plan_t plan);
 
 /* ---- batches of uneven instances -------------------------------------------
  * Many independent 2-D instances of one row-wise template, evaluated by ONE
- * persistent launch (a work queue over row blocks of all instances), which
- * can be replayed as a HIP graph.  Per instance this replaces the plain
+ * persistent launch (row blocks of all instances, balanced over the waves on
+ * the host, the smallest optionally through a work queue), which can be
+ * replayed as a HIP graph.  Per instance this replaces the plain
  * expression sequence
  *   XG_BATCH_SOFTMAX: m = amax(x, {1}, keep_dims); e = exp(x - m);
  *                     out = e / sum(e, {1}, keep_dims)

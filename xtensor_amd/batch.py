@@ -8,7 +8,7 @@ device arrays, the row-wise template
     amax:    out = amax(x, {1})
 
 (xtensor's row softmax of test/test_xmath.cpp:985-1027 and the reducers of
-core/xmath.hpp:1803-1823), and evaluates all of them in one work-queue
+core/xmath.hpp:1803-1823), and evaluates all of them in one persistent
 kernel (`launch()`) or one HIP graph replay (`execute()`).  `autotune()`
 times the candidate launch shapes and caches the choice for the batch's
 shape class.  Inputs need unit column stride; rows may be padded.

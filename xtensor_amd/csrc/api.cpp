@@ -1525,7 +1525,7 @@ xg_status xg_debug_assign_kernel(const xg_expr* e, const xg_tensor* out, char* n
 // Testing aid (host only, no device access): how an assignment past 32-bit
 // offsets is cut.  *n_pieces = the number of pieces (0: not cut), *all_compact
 // = 1 if every piece fits 32-bit offsets, *max_units = the largest piece's
-// work units.  Planned with compiled and run-time compiled programs off.
+// elements (its work units at one element a unit).  Planned with compiled and run-time compiled programs off.
 xg_status xg_debug_assign_pieces(const xg_expr* e, const xg_tensor* out, int64_t* n_pieces, int32_t* all_compact,
                                  int64_t* max_units) {
     return guard([&] {

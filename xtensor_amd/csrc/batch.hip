@@ -212,7 +212,7 @@ constexpr uint32_t kOffNone = 0x80000000u;  // an offset past every resource
 // wave-uniform `lpr_rt`.  One form for them keeps the kernel's instructions at
 // 60 KB: with one per lane count they were 92 KB, more than the 64 KB cache two
 // CUs share, and a batch waited for its code (8 instances, one trip each: 55.9
-// us a launch, 14.7 now; 1024 instances 99.1 -> 45 with the schedule below).
+// us a launch, 8.8 now; 1024 instances 99.1 -> 44.5 with the schedule below).
 template <class T, int OP, int LPR, int NE, int RB>
 __device__ __forceinline__ void rows_regs(const BItem& it, int nrows, int row0, int rb, int sub, int sl, int lpr_rt) {
     using Tr = BTraits<T>;
@@ -495,8 +495,8 @@ int ilog2(double x) { return x < 1.0 ? 0 : int(std::floor(std::log2(x))); }
 
 // Small tasks spread a small batch over the waves, and a purely host-balanced
 // schedule spares every wave its visit to the queue's one counter (float32
-// softmax, default {256, 4, 2048, 10} -> this: 64 instances 68.0 -> 21.5 us,
-// 357 71.6 -> 34.8, 1024 99.1 -> 47.6, 4096 272 -> 223).
+// softmax, default {256, 4, 2048, 10} -> this: 64 instances 68.0 -> 13.1 us,
+// 357 71.6 -> 27.7, 1024 99.1 -> 44.5, 4096 272 -> 215).
 xg_batch_tuning default_tuning() { return xg_batch_tuning{256, 5, 512, 0}; }
 
 void check_tuning(const xg_batch_tuning& t) {

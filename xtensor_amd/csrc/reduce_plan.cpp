@@ -18,7 +18,7 @@ namespace xg {
 
 int g_reduce_waves_per_cu = 16;
 void set_reduce_waves_per_cu(int w) { g_reduce_waves_per_cu = w > 0 ? w : 16; }
-// column fast kernel: 512-thread workgroups per CU, and the split partials'
+// column fast kernel: workgroups (of kColsBlock threads) per CU, and the split partials'
 // share of the input bytes, g_cols_partial_mult / 16
 int g_cols_blocks_per_cu = 1;
 int g_cols_partial_mult = 1;
