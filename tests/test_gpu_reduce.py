@@ -514,3 +514,30 @@ def test_small_expressions_reduce_like_stored_ones(shape, dtype):
             out = xt.empty(got.shape, got.dtype)
             xt.plan(out, f(e, axes)).run()
             assert same_bits(out.to_numpy(), want), (kind, axes)
+
+
+# [outputs' images]: inner rows of 1 element to past a cache line, whole vectors
+# or not, one to many outputs, split and unsplit, none kept, and inside a view
+SHORT_ROWS = [(1000, 50, 3), (200, 64, 4), (37, 5, 16), (64, 3, 31), (9, 1000, 8), (5000, 2, 1), (3000, 4, 2),
+              (100000, 4, 2), (30000, 64, 6), (700, 1, 7), (40, 1000, 33), (2, 6000, 9)]
+
+
+@pytest.mark.parametrize("dtype", ["uint8", "bfloat16", "float32", "float64"])
+@pytest.mark.parametrize("shape", SHORT_ROWS)
+def test_short_inner_rows(dtype, shape):
+    """Integers exact; compensated float sums within one rounding of the oracle's
+    long-double sum, relative to the sum of magnitudes."""
+    rng = np.random.default_rng(sum(shape))
+    h = rng.integers(0, 256, shape).astype("uint8") if dtype == "uint8" else \
+        rng.normal(size=shape).astype("float64" if dtype == "float64" else "float32")
+    d = Dual.of(h, dtype if dtype == "bfloat16" else None)
+    for v in (d, d.view(slice(1, None), slice(None), slice(0, max(1, shape[2] - 1)))):
+        o, r, m = oracle_for(v), xt.sum(v.dev, [0, 2]), xt.amax(v.dev, [0, 2])
+        got = xt.eval(r).to_numpy()
+        if dtype == "uint8":
+            assert same_bits(got, o.reduce(r))
+        else:
+            eps = np.finfo("float64" if dtype == "float64" else "float32").eps
+            mag = o.reduce(xt.sum(xt.abs(v.dev), [0, 2]), high_precision=True)
+            assert np.all(np.abs(got.astype(np.float64) - o.reduce(r, high_precision=True)) <= eps * mag)
+        assert same_bits(xt.eval(m).to_numpy(), o.reduce(m))

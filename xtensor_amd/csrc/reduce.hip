@@ -167,7 +167,9 @@ hipError_t launch_reduce(RedPlan& p, int V, hipStream_t stream, const char** use
             const uint64_t per_block = 4 * (64 / uint64_t(q.group));
             const uint64_t blocks = (items + per_block - 1) / per_block;
             if (blocks >= (uint64_t(1) << 31)) return hipErrorInvalidValue;
+            if (q.f_outputs_first) q.div_splits = make_fastdiv(q.n_out);
             err = go(rows_fast, uint32_t(blocks), 256, q);
+            q.div_splits = make_fastdiv(uint32_t(p.f_splits));
         } else {
             const uint64_t tw = uint64_t(q.group);  // tile width in lanes
             if (tw != 64 && tw != 128 && tw != 256) return hipErrorInvalidValue;

@@ -66,6 +66,7 @@ struct RedPlan {
     uint32_t col_tiles; // RL_COLS: ceil(nchunks_f / 64)
     FastDiv div_col_tiles;
     FastDiv div_splits;
+    int32_t f_outputs_first;  // fast rows of f_rank 3: neighbouring waves take neighbouring outputs, not one's splits
     // finishing: acc -> value type V (vdt) -> [+initial] -> mean / sqrt (rdt) -> out dtype
     int32_t vdt;
     int32_t rdt;

@@ -422,8 +422,11 @@ __global__ __launch_bounds__(256) void reduce_rows_fast_kernel(const RedPlan p) 
     A acc;
     acc.init(p.identity);
     const bool live = wi < items;
-    const uint32_t o = live ? fastdiv(wi, p.div_splits) : 0u;
-    const uint32_t sp = wi - o * uint32_t(p.splits);
+    // RANK 3: div_splits divides by the splits or, with f_outputs_first, by the outputs
+    const uint32_t quot = live ? fastdiv(wi, p.div_splits) : 0u;
+    const uint32_t rem = wi - quot * (RANK == 3 ? p.div_splits.d : uint32_t(p.splits));
+    const bool swap = RANK == 3 && live && p.f_outputs_first != 0;
+    const uint32_t o = swap ? rem : quot, sp = swap ? quot : rem;
     const uint32_t c0 = sp * p.per_split;
     const uint32_t c1 = live ? min(p.red_count, c0 + p.per_split) : 0u;
     // the row and the first element of chunk c
@@ -503,7 +506,7 @@ __global__ __launch_bounds__(256) void reduce_rows_fast_kernel(const RedPlan p) 
     acc = wave_group_combine(acc, G);
     if (live && gl == 0) {
         if (p.splits == 1) finish(p, acc, o);
-        else reinterpret_cast<Store*>(p.partials)[wi] = acc.store();
+        else reinterpret_cast<Store*>(p.partials)[o * uint32_t(p.splits) + sp] = acc.store();
     }
 }
 

@@ -577,7 +577,14 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
     p.div_splits = make_fastdiv(uint32_t(p.splits));
 
     // compact form and the work split of the compiled fast kernels
-    const bool rows3 = p.layout == RL_ROWS && p.n_red == 2 && p.n_kept <= 1;
+    // [outputs | reduced | fast]; rows shorter than a vector are read one a lane
+    // and round there, which pays unless outputs and elements are few (bfloat16
+    // [1000, 50, 3] over its outer dimensions 14.5 us by the general kernel, 16.1
+    // that way, float32 inside a view 7.9 and 10.0; bfloat16 [100, 300, 6] 9.8 and
+    // 5.8, float32 [70001, 2, 2] 11.1 and 10.4, [20000, 50, 3] 28.4 and 17.0)
+    const bool rows3 = p.layout == RL_ROWS && p.n_red == 2 && p.n_kept <= 1 &&
+                       (p.lf >= uint32_t(V) || n_out >= 256 ||
+                        uint64_t(n_out) * (p.red_count / std::max<uint32_t>(p.nchunks_f, 1)) * p.lf >= (uint64_t(1) << 18));
     const bool rows_ok = rows3 || (p.layout == RL_ROWS && p.rank <= 2 && p.n_red == 1);
     const bool cols_ok = p.layout == RL_COLS && p.rank == 2 && p.n_kept == 0;
     if (!p.index64 && (rows_ok || cols_ok) && !empty_red) {
@@ -652,6 +659,14 @@ RedPlan plan_reduce(const xg_expr* e, const xg_reduce_desc* r, const xg_tensor* 
                 p.f_splits = int(s);
             }
         }
+        // Inner rows shorter than a cache line: neighbouring outputs' rows share
+        // lines, so the waves that read them run side by side.  With an output's
+        // splits side by side every line went to several XCDs, at different times:
+        // sums of [n, outputs, row] over n and row, 6 M elements, float32 [., 64, 4]
+        // 31.4 -> 15.8 us, [., 64, 8] 20.5 -> 10.1, float64 [., 1000, 2] 57.5 ->
+        // 23.7, bfloat16 [., 64, 8] 19.5 -> 10.8; from a line up it gives nothing
+        // (float32 rows of 32: 8.0 -> 8.8 over 1000 outputs, 9.4 either way over 64).
+        p.f_outputs_first = rows3 && p.n_kept == 1 && p.f_splits > 1 && uint64_t(p.lf) * 16 < 128 * uint64_t(V) ? 1 : 0;
     }
     return p;
 }
