@@ -79,3 +79,36 @@ def test_gather_and_mixed_conversions():
     b = Dual.of(draw(rng, (300,), "bool"))
     check(xt.cast(b.dev, "int64") + xt.cast(x.dev, "int32") * 2, (b, x))
     check(x.dev * 1.5, (x,), "int8")
+
+
+# either side of the lines between one element a lane and several, for programs
+# that call functions: 2^18 elements, and 2^19 for 32-bit ones of mostly calls
+@pytest.mark.parametrize("n", [1, 63, 1000, (1 << 18) - 1, 1 << 18, (1 << 19) - 1, (1 << 19) + 1])
+@pytest.mark.parametrize("dtype", ["int8", "uint16", "int32", "int64"])
+def test_called_ops_by_size(n, dtype):
+    """Integer divisions and remainders (called), bit for bit; a contiguous
+    output, one inside a larger array, and operands that are views."""
+    rng = np.random.default_rng(n)
+    a, b = (Dual.of(rng.integers(1, 100, n + 3).astype(dtype)) for _ in range(2))
+    av, bv = a.view(slice(1, n + 1)), b.view(slice(2, n + 2))
+    e = (av.dev / bv.dev) + (av.dev % bv.dev) * (bv.dev % av.dev)
+    want = oracle_for(av, bv).assign(e)
+    assert same_bits(xt.eval(e).to_numpy(), want)
+    whole = xt.from_numpy(np.full(n + 2, 7, want.dtype))
+    xt.noalias(whole[1:-1]).assign(e)
+    got = whole.to_numpy()
+    assert same_bits(got[1:-1], want) and got[0] == 7 and got[-1] == 7
+
+
+@pytest.mark.parametrize("n", [1, 1000, (1 << 18) - 1, (1 << 19) - 1, (1 << 19) + 1])
+def test_gather_and_many_leaves_by_size(n):
+    rng = np.random.default_rng(n)
+    x = Dual.of(rng.normal(size=500).astype(np.float32))
+    i = Dual.of(rng.integers(0, 500, n).astype(np.int64))
+    g = xt.index_view(x.dev, i.dev)
+    assert same_bits(xt.eval(g * np.float32(2)).to_numpy(), x.host[i.host] * np.float32(2))
+    ls = [Dual.of(rng.normal(size=n).astype(np.float32)) for _ in range(9)]
+    e, want = ls[0].dev, ls[0].host
+    for l in ls[1:]:
+        e, want = e + l.dev, want + l.host
+    assert same_bits(xt.eval(e).to_numpy(), want)

@@ -26,7 +26,8 @@ namespace xg {
 //     integer division, gathers, many leaves) keep theirs in functions that
 //     are called.
 // W64 = false: programs without a 64-bit type, whose registers are 32 bits
-// wide and carry V = 4 elements; otherwise V = 2.  Float32 standardisation
+// wide and carry V = 4 elements; otherwise V = 2; V = 1 for few elements of a
+// program that calls (ew_interp_width).  Float32 standardisation
 // (five leaves, nine ops) of [1013, 771]: 21.8 us a launch with one element a
 // lane, registers in LDS and an out-of-line call per op, 9.2 us now (float64 22.0 ->
 // 13.2; the headline expression forced through it 1.82 -> 0.61 ms).
@@ -59,7 +60,7 @@ __device__ __forceinline__ void load_raw_chunk(const char* p, int dt, int mode, 
                                                uint32_t (&w)[4]) {
     const int esz = dtype_size(dt);
     w[0] = w[1] = w[2] = w[3] = 0;
-    if (mode == LM_BCAST) {
+    if (V == 1 || mode == LM_BCAST) {
         const uint64_t x = load_raw(p, esz);
         w[0] = uint32_t(x);
         w[1] = uint32_t(x >> 32);
@@ -357,8 +358,8 @@ __global__ __launch_bounds__(256) void ew_interp_kernel(const EwPlan plan_arg) {
         file.get(plan.prog.result_reg, res);
         const int odt = plan.out_dtype, esz = dtype_size(odt);
         char* p = plan.out_ptr + offset(kMaxLeaves) * esz;
-        if (lm_base(plan.out_mode) == LM_CONTIG && nvalid == V) {
-            store_vec<V>(p, esz, odt, res);
+        if (V > 1 && lm_base(plan.out_mode) == LM_CONTIG && nvalid == V) {
+            if constexpr (V > 1) store_vec<V>(p, esz, odt, res);
         } else {
             const int64_t os = plan.out_stride[rank - 1] * esz;
 #pragma unroll
@@ -368,11 +369,8 @@ __global__ __launch_bounds__(256) void ew_interp_kernel(const EwPlan plan_arg) {
     }
 }
 
-// LIGHT: every op is one light_op takes, and the leaves fit the registers
-bool interp_light(const EwPlan& p) {
-    if (p.prog.nleaves > kInterpPre) return false;
-    for (int l = 0; l < p.prog.nleaves; ++l)
-        if (p.prog.leaf_gather[l]) return false;
+// ops that light_op does not take
+int called_ops(const EwPlan& p) {
     auto cvt_ok = [](int from, int to) {
 #define XG_CVT(FROM, TO) if (from == FROM && to == TO) return true;
         XG_LIGHT_CVT32
@@ -380,27 +378,30 @@ bool interp_light(const EwPlan& p) {
 #undef XG_CVT
         return false;
     };
-    for (int i = 0; i < p.prog.nops; ++i) {
-        const MicroOp& m = p.prog.ops[i];
+    auto light = [&](const MicroOp& m) {
         switch (m.op) {
-        case MO_LOAD: case MO_CONST: case MO_LNOT: case MO_LAND: case MO_LOR: case MO_SEL: continue;
-        case MO_CVT:
-            if (!cvt_ok(m.t, m.aux)) return false;
-            continue;
+        case MO_LOAD: case MO_CONST: case MO_LNOT: case MO_LAND: case MO_LOR: case MO_SEL: return true;
+        case MO_CVT: return cvt_ok(m.t, m.aux);
         case MO_ADD: case MO_SUB: case MO_MUL: case MO_LT: case MO_LE: case MO_GT: case MO_GE: case MO_EQ: case MO_NE:
-            if (m.t != XG_FLOAT32 && m.t != XG_FLOAT64 && m.t != XG_INT32 && m.t != XG_INT64) return false;
-            continue;
+            return m.t == XG_FLOAT32 || m.t == XG_FLOAT64 || m.t == XG_INT32 || m.t == XG_INT64;
         case MO_DIV: case MO_NEG: case MO_ABS: case MO_EXP: case MO_LOG: case MO_SQRT: case MO_FLOOR: case MO_CEIL:
         case MO_TRUNC: case MO_ROUND:
-            if (m.t != XG_FLOAT32 && m.t != XG_FLOAT64) return false;
-            continue;
-        case MO_BAND: case MO_BOR: case MO_BXOR: case MO_SHL: case MO_SHR:
-            if (m.t != XG_INT32 && m.t != XG_INT64) return false;
-            continue;
+            return m.t == XG_FLOAT32 || m.t == XG_FLOAT64;
+        case MO_BAND: case MO_BOR: case MO_BXOR: case MO_SHL: case MO_SHR: return m.t == XG_INT32 || m.t == XG_INT64;
         default: return false;
         }
-    }
-    return true;
+    };
+    int n = 0;
+    for (int i = 0; i < p.prog.nops; ++i) n += light(p.prog.ops[i]) ? 0 : 1;
+    return n;
+}
+
+// LIGHT: every op is one light_op takes, and the leaves fit the registers
+bool interp_light(const EwPlan& p) {
+    if (p.prog.nleaves > kInterpPre) return false;
+    for (int l = 0; l < p.prog.nleaves; ++l)
+        if (p.prog.leaf_gather[l]) return false;
+    return called_ops(p) == 0;
 }
 
 using InterpFn = void (*)(const EwPlan);
@@ -410,23 +411,44 @@ template <int V, bool W64> InterpFn interp_kernel(bool compact, bool light) {
     return compact ? ew_interp_kernel<V, W64, true, false> : ew_interp_kernel<V, W64, false, false>;
 }
 
-// Elements per lane: four when nothing in the program or its operands is 64
-// bits wide, else two.
-int ew_interp_width(const EwPlan& p) {
-    if (dtype_size(p.out_dtype) == 8) return 2;
+// one element a lane: the programs that call
+InterpFn interp_kernel_1(bool compact, bool w64) {
+    if (w64) return compact ? ew_interp_kernel<1, true, true, false> : ew_interp_kernel<1, true, false, false>;
+    return compact ? ew_interp_kernel<1, false, true, false> : ew_interp_kernel<1, false, false, false>;
+}
+
+// something in the program or its operands is 64 bits wide
+bool interp_64(const EwPlan& p) {
+    if (dtype_size(p.out_dtype) == 8) return true;
     for (int l = 0; l < p.prog.nleaves; ++l)
-        if (p.prog.leaf_gather[l] || dtype_size(p.leaves[l].dtype) == 8) return 2;
+        if (p.prog.leaf_gather[l] || dtype_size(p.leaves[l].dtype) == 8) return true;
     for (int i = 0; i < p.prog.nops; ++i) {
         const MicroOp& m = p.prog.ops[i];
-        if (m.op == MO_GATHER || (m.op != MO_LOAD && is_64bit(m.t)) || (m.op == MO_CVT && is_64bit(m.aux))) return 2;
+        if (m.op == MO_GATHER || (m.op != MO_LOAD && is_64bit(m.t)) || (m.op == MO_CVT && is_64bit(m.aux))) return true;
     }
-    return 4;
+    return false;
+}
+
+// Elements per lane.  Light programs: four when nothing is 64 bits wide, else
+// two.  The others call a function per op and element, one after the other in a
+// lane: with few elements, whose waves do not fill the GPU, they take one a
+// lane (float32 tanh(sin(a) + cos(b)) * erf(a) + atan(b) of 30,000 elements
+// 20.8 us with four, 9.7 with one; of 400,000 22.8 and 18.1; of 900,000 29.0
+// and 30.6; float64 of 120,000 15.0 and 11.2, of 400,000 21.6 and 22.7; nine
+// float32 leaves added, of 250,000 15.6 and 13.3, of 400,000 15.8 and 20.1).
+int ew_interp_width(const EwPlan& p) {
+    const bool w64 = interp_64(p);
+    const uint64_t n = p.nchunks ? p.units / p.nchunks * p.inner : 0;
+    if (n < (uint64_t(1) << 19) && !interp_light(p) &&
+        (n < (uint64_t(1) << 18) || (!w64 && called_ops(p) * 4 >= p.prog.nops)))
+        return 1;
+    return w64 ? 2 : 4;
 }
 
 hipError_t launch_ew_interp(const EwPlan& p, int V, dim3 grid, hipStream_t stream) {
     if (V != ew_interp_width(p)) return hipErrorInvalidValue;
     const bool light = interp_light(p);
-    InterpFn f = V == 4 ? interp_kernel<4, false>(p.compact != 0, light) : interp_kernel<2, true>(p.compact != 0, light);
+    InterpFn f = V == 1 ? interp_kernel_1(p.compact != 0, interp_64(p)) : V == 4 ? interp_kernel<4, false>(p.compact != 0, light) : interp_kernel<2, true>(p.compact != 0, light);
     hipLaunchKernelGGL(f, grid, dim3(256), 0, stream, p);
     return hipGetLastError();
 }
