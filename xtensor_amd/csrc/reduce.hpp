@@ -66,7 +66,6 @@ struct RedPlan {
     uint32_t col_tiles; // RL_COLS: ceil(nchunks_f / 64)
     FastDiv div_col_tiles;
     FastDiv div_splits;
-    int32_t f_outputs_first;  // fast rows of f_rank 3: neighbouring waves take neighbouring outputs, not one's splits
     // finishing: acc -> value type V (vdt) -> [+initial] -> mean / sqrt (rdt) -> out dtype
     int32_t vdt;
     int32_t rdt;
@@ -97,6 +96,7 @@ struct RedPlan {
     int32_t f_group;      // rows: lanes per output (1..64, power of two); cols: tile width in lanes (64, 128, 256)
     int32_t f_splits;     // partial results per output
     uint32_t f_per_split; // rows: chunks per split; cols: rows per split
+    int32_t f_outputs_first;  // rows of f_rank 3: neighbouring waves take neighbouring outputs, not one's splits
     int32_t cst[kMaxLeaves + 1][4];
 };
 
